@@ -487,25 +487,52 @@ AH_DEV void ffn_epilogue(const FfnArgs &fa, uint32_t b0, uint32_t b1, const floa
 // 32-lane half-wave per (token, hidden block), the wave's two blocks consecutive; refusals keyed
 // past the projections': an element's conversion or SwiGLU at key_sw + t * n_ff + k, a block's
 // quantizer at key_q + t * ceil(n_ff / 32) + b.
+// Bound by its f64 arithmetic (about 130 VALU instructions an element; the 9 bytes an element
+// move faster).  A wave steps by the whole grid, so its (token, block) advances by a fixed pair
+// with one carry instead of a division, and its next two blocks are requested before it computes.
 __global__ void __launch_bounds__(kThreads) swiglu_quant_kernel(SwigluArgs a) {
     const uint32_t nbh = (a.n_ff + 31) / 32;
-    const uint64_t total = (uint64_t)a.n_tok * nbh;
     const uint32_t lane = threadIdx.x & 63u, l = lane & 31u, half = lane >> 5;
-    const uint64_t wave = ((uint64_t)blockIdx.x * kThreads + threadIdx.x) / 64;
-    const uint64_t waves = (uint64_t)gridDim.x * (kThreads / 64);
-    for (uint64_t p = wave; 2 * p < total; p += waves) {  // the same trip count for the whole wave
-        const uint64_t blk = 2 * p + half;
-        const bool vb = blk < total;
-        const uint32_t t = vb ? (uint32_t)(blk / nbh) : 0u, b = vb ? (uint32_t)(blk % nbh) : 0u;
-        const uint32_t k = 32u * b + l;
-        const bool live = vb && k < a.n_ff;
-        const size_t e = (size_t)t * a.n_ff + k;
-        const uint32_t gb = live ? __builtin_bit_cast(uint32_t, a.gate[e]) : 0u;
-        const uint32_t ub = live ? __builtin_bit_cast(uint32_t, a.up[e]) : 0u;
-        const HiddenQ q = swiglu_quant32(gb, ub, live);
+    const uint32_t w2 = 2 * __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + threadIdx.x / 64);
+    const uint32_t step = 2 * gridDim.x * (kThreads / 64), step_t = step / nbh, step_b = step - step_t * nbh;
+    uint32_t t0 = w2 / nbh, b0 = w2 - t0 * nbh;  // the wave's first block (uniform)
+    struct In {
+        uint32_t t, b, g, u;
+        bool live;
+    };
+    auto fetch = [&](uint32_t tw, uint32_t bw) {
+        In in;
+        in.b = bw + half;
+        in.t = tw;
+        if (in.b >= nbh) {
+            in.b -= nbh;
+            ++in.t;
+        }
+        const uint32_t k = 32u * in.b + l;
+        in.live = in.t < a.n_tok && k < a.n_ff;
+        // (a dead lane reads element 0: loads behind a branch would be waited for at once)
+        const size_t e = in.live ? (size_t)in.t * a.n_ff + k : 0;
+        in.g = __builtin_bit_cast(uint32_t, a.gate[e]);
+        in.u = __builtin_bit_cast(uint32_t, a.up[e]);
+        return in;
+    };
+    In next = fetch(t0, b0);
+    while (t0 < a.n_tok) {  // the same trip count for the whole wave
+        const In in = next;
+        t0 += step_t;
+        b0 += step_b;
+        if (b0 >= nbh) {
+            b0 -= nbh;
+            ++t0;
+        }
+        next = fetch(t0, b0);
+        const uint32_t k = 32u * in.b + l;
+        const size_t e = (size_t)in.t * a.n_ff + k;
+        const HiddenQ q = swiglu_quant32(in.g, in.u, in.live);
         if (q.err) ah_record(a.status, ah_out_key(a.key_sw + e, (uint32_t)q.err));
-        if (live) a.h_codes[e] = (int8_t)q.code;
-        if (vb && l == 0) {
+        if (in.live) a.h_codes[e] = (int8_t)q.code;
+        if (in.live && l == 0) {
+            const size_t blk = (size_t)in.t * nbh + in.b;
             if (q.bad_block) ah_record(a.status, ah_out_key(a.key_q + blk, 7u));
             a.h_scales[blk] = (int64_t)q.scale;
         }
@@ -1382,7 +1409,7 @@ hipError_t ah_launch_swiglu_quant(const SwigluArgs &a, hipStream_t stream) {
     const uint64_t total = (uint64_t)a.n_tok * ((a.n_ff + 31) / 32);
     if (total == 0) return hipSuccess;
     uint64_t grid = (total + 7) / 8;  // 8 blocks per 256-thread workgroup
-    if (grid > 8192) grid = 8192;
+    if (grid > 2048) grid = 2048;     // 8 workgroups a CU: every wave slot at 64 VGPRs
     hipLaunchKernelGGL(swiglu_quant_kernel, dim3((uint32_t)grid), dim3(kThreads), 0, stream, a);
     return hipGetLastError();
 }

@@ -260,3 +260,31 @@ def test_swiglu_quant_dev_vs_oracle(dev):
     dg, du = torch.from_numpy(g).cuda(), torch.from_numpy(u).cuda()
     chart.swiglu_quant_dev(dev, dg.data_ptr(), du.data_ptr(), n_tok, n_ff, hc.data_ptr(), hs.data_ptr(), stream())
     assert dev.sync_status(stream()) == oracle.swiglu_quant_f32(g[3], u[3])[0] == 12
+
+
+@pytest.mark.parametrize("scale_g,scale_u", [(0.25, 1.0), (8.0, 8.0), (40.0, 300.0), (400.0, 900.0)])
+def test_swiglu_quant_f64_form_and_its_edges(dev, scale_g, scale_u):
+    """Waves wholly inside the f64 form's range, waves with one lane past either bound, exact ties of
+    the exp's Horner products (gates that are small powers of two), saturated and zero gates, a
+    partial last block: the hidden QuantAct equals the oracle's integers."""
+    rng = np.random.default_rng(int(scale_g * 8))
+    n_tok, n_ff = 24, 333
+    g = (rng.standard_normal((n_tok, n_ff)) * scale_g).astype(np.float32)
+    u = (rng.standard_normal((n_tok, n_ff)) * scale_u).astype(np.float32)
+    edge = np.float32([512.0, np.nextafter(np.float32(512), np.float32(0)), 16.0, np.nextafter(np.float32(16), np.float32(0)),
+                       -21.0, np.nextafter(np.float32(-21), np.float32(0)), 0.0, -0.0, 2.0 ** -33, 1.5 * 2.0 ** -33])
+    for i, v in enumerate(edge):
+        g[i, 31 * i + 5] = v
+        u[i, 29 * i + 7] = v * 2
+    g[12, ::3] = np.ldexp(np.float32(1), rng.integers(-8, 3, g[12, ::3].shape).astype(np.int32)) * np.where(rng.random(g[12, ::3].shape) < 0.5, -1, 1)
+    g[13], u[14] = 0, 0
+    u[15, 100] = 1024.0
+    hc = torch.zeros((n_tok, n_ff), dtype=torch.int8, device="cuda")
+    hs = torch.zeros((n_tok, 11), dtype=torch.int64, device="cuda")
+    dg, du = torch.from_numpy(g).cuda(), torch.from_numpy(u).cuda()
+    chart.swiglu_quant_dev(dev, dg.data_ptr(), du.data_ptr(), n_tok, n_ff, hc.data_ptr(), hs.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0
+    HC, HS = hc.cpu().numpy(), hs.cpu().numpy()
+    for t in range(n_tok):
+        st, codes, scales, _ = oracle.swiglu_quant_f32(g[t], u[t])
+        assert st == 0 and (HC[t] == codes).all() and (HS[t] == scales).all(), t

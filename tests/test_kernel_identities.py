@@ -10,6 +10,9 @@
   cleared below half a code unit, a second rounding below 2^-9 at exponents <= 24), against
   quant_act_f32, with a brute force over every f32 of the fma's sum.
 """
+import math
+from fractions import Fraction
+
 import numpy as np
 
 import oracle
@@ -279,3 +282,63 @@ def test_silu_single_correction_is_exact():
         got, off = silu_one_step(v)
         st, ref = oracle.silu_fixed(v)
         assert st == 0 and got == ref and abs(off) <= 1, (v, off)
+
+
+# ---- the SwiGLU's f64 form (swiglu_quant32_f64 in ah_swiglu.h) ------------------------------------
+
+
+def _fma(a: float, b: float, c: float) -> float:
+    """One rounding (nearest, ties to even: Fraction's conversion) of the exact a * b + c."""
+    return float(Fraction(a) * Fraction(b) + Fraction(c))
+
+
+def swiglu_f64(gq: int, uq: int):
+    """swiglu_quant32_f64's h from Q32.32 gate and up values inside its range, step for step (every
+    operation one f64 rounding), with the quotient estimate off by up to `2^-44` either way; None
+    where a Horner product is a tie (the kernel then takes the integer form)."""
+    M, g, u = 6755399441055744.0, float(gq), float(uq)
+    x = min(max(-g, -(2.0 ** 36)), 21.0 * 2.0 ** 32)
+    kd = float(math.floor(_fma(x, 6196328019.0 * 2.0 ** -64, 0.5)))
+    assert int(kd) == (int(x) * 6196328019 + (1 << 63)) >> 64, gq
+    r = _fma(kd, -2977044472.0, x)
+    rs, acc = r * 2.0 ** -32, 852176.0
+    for c in _EXP_C[1:]:
+        m = _fma(acc, rs, M)
+        if abs(_fma(acc, rs, M - m)) == 0.5:
+            return None
+        acc = m - (M - float(c))
+    den = float(math.floor(math.ldexp(acc, int(kd)) + 0.5)) + 2.0 ** 32
+    hd = float(math.floor(0.5 * den))
+    out = set()
+    for off in (-1.0, 0.0, 1.0):
+        est = float(Fraction(abs(g) * 2.0 ** 32) / Fraction(den)) * (1.0 + off * 2.0 ** -44)
+        q = float(round(est))
+        rem = _fma(-q, den, abs(g) * 2.0 ** 32)
+        assert Fraction(rem) == Fraction(abs(g) * 2.0 ** 32) - Fraction(q) * Fraction(den)
+        q += -1.0 if rem < -hd else 1.0 if rem >= den - hd else 0.0
+        s = g if g >= 2.0 ** 36 else 0.0 if g <= -21.0 * 2.0 ** 32 else math.copysign(q, g)
+        us = u * 2.0 ** -32
+        m = _fma(s, us, M)
+        out.add((m - M) + (1.0 if _fma(s, us, M - m) == 0.5 else 0.0))
+    assert len(out) == 1
+    return int(out.pop())
+
+
+def test_swiglu_f64_equals_integer_form():
+    """swiglu_quant32_f64's value is the oracle's i128 swiglu over its whole range: the range
+    reduction's half-way points and their neighbours at every k (where k's rounding is closest),
+    the saturation bounds, products that are exact halves, the ends of the range and a sweep."""
+    one, ln2 = 1 << 32, 2977044472
+    g = [0, 1, -1, 16 * one - 1, 16 * one, -21 * one, -21 * one + 1, (one << 9) - (1 << 17), -(one << 9) + (1 << 17)]
+    for k in range(-24, 32):
+        g += [-((2 * k + 1) * ln2 // 2 + d) for d in range(-2, 4)]
+    rng = np.random.default_rng(0xF64)
+    g += [int(v) for v in rng.integers(-21 * one, 16 * one, size=1500)] + [int(v) for v in rng.integers(-one, one, size=500)]
+    u = [one, one >> 1, -(one >> 1), 3 << 30, 1, (one << 10) - (1 << 18), -(one << 10) + (1 << 18)]
+    ties = 0
+    for i, v in enumerate(g):
+        for w in (u[i % len(u)], int(rng.integers(-8 * one, 8 * one))):
+            got = swiglu_f64(v, w)
+            ties += got is None
+            assert got is None or oracle.swiglu(v, w) == (0, got), (v, w)
+    assert ties < len(g) // 20

@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libapeiron_hip.so")
-SOURCES = ["ah_gemv.hip", "ah_gemm.hip", "ah_abi.cpp"]
+SOURCES = ["ah_gemv.hip", "ah_gemm.hip", "ah_few.hip", "ah_abi.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",

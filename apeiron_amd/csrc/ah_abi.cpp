@@ -4,6 +4,7 @@
 // geometry exactly like matvec_fixed (ops/matvec.rs:160-175), scans f16 block scales for the
 // NonFiniteScale refusal (num/dequant.rs:25-41), and plans the kernel launches.
 #include "apeiron_hip.h"
+#include "ah_few.h"
 #include "ah_internal.h"
 
 #include <hip/hip_runtime.h>
@@ -55,6 +56,10 @@ uint32_t ah_gemm_max_parts(uint32_t type);
 uint32_t ah_gemm_pick_waves(uint32_t type, uint64_t n_wg4, uint32_t cus, bool int8);
 hipError_t ah_launch_gemm_operand(const OperandArgs &o, hipStream_t stream);
 hipError_t ah_launch_swiglu_quant(const SwigluArgs &a, hipStream_t stream);
+size_t ah_few_lds_bytes(uint32_t type, uint32_t kpad, uint32_t tok, uint32_t waves);
+uint32_t ah_few_splits(uint32_t type, uint32_t n_in);
+hipError_t ah_few_init_attrs();
+hipError_t ah_launch_few(uint32_t type, FewArgs &a, bool ffn, hipStream_t stream);
 hipError_t ah_probe_mfma(uint32_t kind, uint32_t cus, const uint32_t *d_seed, uint32_t *d_sink,
                          hipStream_t stream, double *tops);
 
@@ -485,6 +490,85 @@ int32_t reset_status(ah_ctx *ctx) {
     return AH_OK;
 }
 
+// The few-token route (ah_few.hip): calls of at most kFewTokens tokens whose type's design is AUTO.
+// Its tokens per workgroup (all of them up to 32, as far as their quantized rows fit a CU's LDS); 0:
+// the call takes the tile GEMM.  At most two token tiles: each streams the weights again, and from
+// the third on the tile GEMM is faster (Q4_K 1536 x 8960 from codes, tiles of 8 tokens: 14.3 us
+// against 24.1 at 16 tokens, 24.9 against 20.1 at 24).  Past 16 tokens a family with min terms takes
+// the tile GEMM once its rows fill the device (from f32, 32 tokens: Q4_K 8960 x 1536 19.6 us against
+// 17.7, 896 x 896 13.1 against 15.2; Q8_0 8960 x 1536 17.9 against 26.1).
+constexpr size_t kFewTokens = 32;
+uint32_t few_tok_tile(const ah_ctx *ctx, const ah_tensor *t, size_t n_tok) {
+    if (n_tok > kFewTokens || ctx->design[t->type] != AH_GEMM_DESIGN_AUTO) return 0;
+    if (n_tok > 16 && (t->type == AH_GGML_Q4_K || t->type == AH_GGML_Q2_K) && t->n_out > 16 * (size_t)ctx->cu_count) return 0;
+    uint32_t tok = n_tok > 16 ? 32u : 16u;
+    while (tok >= 8 && ah_few_lds_bytes(t->type, kpad_of(t->n_in), n_tok < tok ? (uint32_t)n_tok : tok, kFewMaxWaves) > 160 * 1024)
+        tok /= 2;
+    return tok >= 8 && n_tok <= 2 * tok ? tok : 0;
+}
+FewArgs few_args(uint32_t src, const void *x, const int64_t *scales, uint32_t n_in, uint32_t n_tok, uint32_t tok_tile,
+                 unsigned long long *status) {
+    FewArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.x = x;
+    a.scales = scales;
+    a.status = status;
+    a.n_in = n_in;
+    a.n_tok = n_tok;
+    a.kpad = kpad_of(n_in);
+    a.src = src;
+    a.pitch = n_in;
+    a.bytewise = src == AH_SRC_CODES && (n_in % 4 || reinterpret_cast<uintptr_t>(x) % 4) ? 1u : 0u;
+    a.tok_tile = tok_tile;
+    return a;
+}
+// An f32 input that every workgroup would quantize in more than kFewPasses passes over its threads
+// (about 0.7 us each) is quantized once by a launch of its own (3.5 us) into scratch instead: Q4_K
+// 8960 x 1536 at 16 tokens took 18.2 us against 11.5 from codes, at 8 tokens 13.2 against 10.4.
+constexpr uint32_t kFewPasses = 5;
+int32_t few_quantize(ah_ctx *ctx, FewArgs &a, void *stream, uint8_t *fixed, size_t fixed_cap) {
+    const uint32_t tok = a.n_tok < a.tok_tile ? a.n_tok : a.tok_tile;
+    if (a.src != AH_SRC_F32 || (uint64_t)tok * (a.kpad / 32) <= (uint64_t)kFewPasses * 16 * a.waves) return AH_OK;
+    const uint32_t pitch = (a.n_in + 15u) & ~15u, nb32 = (a.n_in + 31) / 32;
+    const size_t o_s = align256((size_t)a.n_tok * pitch), need = o_s + (size_t)a.n_tok * nb32 * 8;
+    uint8_t *S = fixed;
+    if (fixed) {
+        if (need > fixed_cap) return AH_ERR_SCRATCH_LIMIT;
+    } else {
+        const int32_t st = ensure_scratch(ctx, need);
+        if (st) return st;
+        S = static_cast<uint8_t *>(ctx->scratch);
+    }
+    QuantArgs q;
+    q.x = a.x;
+    q.codes = reinterpret_cast<int8_t *>(S);
+    q.scales = reinterpret_cast<int64_t *>(S + o_s);
+    q.n_tok = a.n_tok;
+    q.n_in = a.n_in;
+    q.nb32 = nb32;
+    q.pitch = pitch;
+    q.src = AH_SRC_F32;
+    q.status = a.status;
+    AH_HIP(ctx, hipSetDevice(ctx->device));
+    AH_HIP(ctx, ah_launch_quant(q, pick(ctx, stream)));
+    a.x = q.codes;
+    a.scales = q.scales;
+    a.src = AH_SRC_CODES;
+    a.pitch = pitch;
+    return AH_OK;
+}
+FewPart few_part(const ah_tensor *t, float *y, uint64_t key0) {
+    FewPart p;
+    p.w = t->d;
+    p.y = y;
+    p.w_bytes = (uint32_t)t->bytes;
+    p.row_bytes = (uint32_t)t->row_bytes;
+    p.n_out = (uint32_t)t->n_out;
+    p.wg_begin = 0;
+    p.key0 = key0;
+    return p;
+}
+
 // GEMM operand preparation + launch.  src = AH_SRC_F32 (x = f32 [n_tok][n_in]) or AH_SRC_CODES.
 // Prefill over n_parts projections of one input: one operand pass (shared by every part, as the
 // reference's grouped GEMM shares one activation pack, kern/gemm.rs:799-818), then one GEMM launch
@@ -561,8 +645,46 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
     // the other parts then go through the GEMM below.  Nothing is allocated on this route (parts
     // past kStackParts aside).  By default these families take the dequantize-once MFMA tiles.
     auto gemv23 = [&](const ah_tensor *t) { return ah_k23((int)t->type) && kind_of(t->type) != kGemmKindTile; };
-    size_t n23 = 0;
-    for (size_t i = 0; i < n_parts; ++i) n23 += gemv23(w[i]) ? 1 : 0;
+    size_t n23 = 0, n_few = 0;
+    // Few-token parts: one launch per run of parts of one type.  (The fused FFN form
+    // and a part without rows stay below.)
+    auto few = [&](const ah_tensor *t) { return !ffn && t->n_out ? few_tok_tile(ctx, t, n_tok) : 0u; };
+    auto direct = [&](const ah_tensor *t) { return few(t) != 0 || gemv23(t); };
+    for (size_t i = 0; i < n_parts; ++i) {
+        n_few += few(w[i]) ? 1 : 0;
+        n23 += !few(w[i]) && gemv23(w[i]) ? 1 : 0;
+    }
+    if (n_few) {
+        AH_HIP(ctx, hipSetDevice(ctx->device));
+        FewArgs q = {};  // the input once quantized
+        for (size_t i = 0; i < n_parts;) {
+            const uint32_t tile = few(w[i]);
+            if (!tile) {
+                ++i;
+                continue;
+            }
+            const uint32_t type = w[i]->type;
+            FewArgs fa = few_args(src, x, scales_in, (uint32_t)n_in_sz, (uint32_t)n_tok, tile, status);
+            fa.splits = ah_few_splits(type, fa.n_in);
+            fa.waves = fa.splits >= 8 ? fa.splits : 8 / fa.splits * fa.splits;
+            for (; i < n_parts && fa.n_parts < kFewMaxParts; ++i) {
+                if (w[i]->n_out == 0) continue;
+                if (w[i]->type != type || few(w[i]) != tile) break;
+                fa.p[fa.n_parts++] = few_part(w[i], y[i], key0[i]);
+            }
+            if (q.x) {
+                fa.x = q.x;
+                fa.scales = q.scales;
+                fa.src = q.src;
+                fa.pitch = q.pitch;
+            } else {
+                const int32_t st = few_quantize(ctx, fa, stream, fixed, fixed_cap);
+                if (st) return st;
+                if (fa.src != src) q = fa;
+            }
+            AH_HIP(ctx, ah_launch_few(type, fa, false, pick(ctx, stream)));
+        }
+    }
     if (n23) {
         const size_t nb = (n_in_sz + 31) / 32;
         // the GEMV reads codes a dword at a time: token rows of codes whose length is not a multiple
@@ -587,7 +709,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
         const uint32_t kp = kpad_of(n_in_sz);
         AH_HIP(ctx, hipSetDevice(ctx->device));
         for (size_t i = 0; i < n_parts; ++i) {
-            if (!gemv23(w[i]) || w[i]->n_out == 0) continue;
+            if (few(w[i]) || !gemv23(w[i]) || w[i]->n_out == 0) continue;
             // rows that fit the streaming kernel's tile: four tokens per launch, as the argument
             // parts of one launch (each workgroup quantizes its own token's activation), so each
             // launch fills more of the device and the weight rows are re-read from L2
@@ -618,7 +740,11 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
                 c += sp.n;
             }
         }
-        if (n23 == n_parts) return AH_OK;
+    }
+    if (n_few || n23) {
+        size_t n_rest = 0;
+        for (size_t i = 0; i < n_parts; ++i) n_rest += !direct(w[i]) && w[i]->n_out ? 1 : 0;
+        if (n_few ? n_rest == 0 : n23 == n_parts) return AH_OK;
         const ah_tensor *rw_stack[kStackParts];
         float *ry_stack[kStackParts];
         std::vector<const ah_tensor *> rw_heap;
@@ -632,7 +758,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
         float **ry = n_parts > kStackParts ? ry_heap.data() : ry_stack;
         size_t k = 0;
         for (size_t i = 0; i < n_parts; ++i)
-            if (!gemv23(w[i])) {
+            if (!direct(w[i])) {
                 rw[k] = w[i];
                 ry[k++] = y[i];
             }
@@ -644,7 +770,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
         uint64_t *t0 = n_parts > kStackParts ? t_heap.data() : t_stack;
         size_t q = 0;
         for (size_t i = 0; i < n_parts; ++i)
-            if (!gemv23(w[i])) t0[q++] = key0[i];
+            if (!direct(w[i])) t0[q++] = key0[i];
         o2.key0 = t0;
         return gemm_group_launch(ctx, k, rw, src, x, scales_in, n_tok, ry, stream, fixed, fixed_cap, &o2);
     }
@@ -872,7 +998,7 @@ int32_t ah_init(int32_t device, ah_ctx **out) {
     ctx->cu_count = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&ctx->stream) != hipSuccess ||
         hipMalloc(&ctx->d_status, 2 * sizeof(unsigned long long)) != hipSuccess ||
-        ah_gemv_init_attrs() != hipSuccess) {
+        ah_gemv_init_attrs() != hipSuccess || ah_few_init_attrs() != hipSuccess) {
         delete ctx;
         return AH_ERR_HIP;
     }
@@ -1046,6 +1172,7 @@ static int32_t quant_dev(ah_ctx *ctx, uint32_t src, const void *d_x, size_t n_to
     q.n_tok = (uint32_t)n_tok;
     q.n_in = (uint32_t)n_in;
     q.nb32 = (uint32_t)((n_in + 31) / 32);
+    q.pitch = q.n_in;
     q.src = src;
     q.status = ctx->d_status;
     AH_HIP(ctx, hipSetDevice(ctx->device));
@@ -1190,6 +1317,27 @@ static int32_t ffn_prefill_gate_up(ah_ctx *ctx, const ah_tensor *gate, const ah_
         GroupOpts o;
         o.ffn = &f;
         return gemm_group_launch(ctx, 2, w2, src, d_x, d_scales, n_tok, y2, stream, nullptr, 0, &o);
+    }
+    if (n_ff > (0xFFFFFF00ull / (128 * 4))) return AH_ERR_INVALID_ARG;  // as gemm_group_launch refuses it
+    // a few tokens: one launch, the SwiGLU in its epilogue (a workgroup is the K splits of two row
+    // tiles of each projection, so at most four splits)
+    const uint32_t ffn_splits = ah_few_splits(t, (uint32_t)gate->n_in);
+    if (const uint32_t tile = ctx->ffn_form == AH_FFN_PREFILL_AUTO && 4 * ffn_splits <= kFewMaxWaves ? few_tok_tile(ctx, gate, n_tok) : 0) {
+        FewArgs fa = few_args(src, d_x, d_scales, (uint32_t)gate->n_in, (uint32_t)n_tok, tile, ctx->d_status);
+        fa.n_parts = 2;
+        fa.p[0] = few_part(gate, nullptr, 0);
+        fa.p[1] = few_part(up, nullptr, 0);
+        fa.splits = ffn_splits;
+        fa.waves = 4 * fa.splits;
+        fa.gy = d_gate_y;
+        fa.uy = d_up_y;
+        fa.h_codes = d_h_codes;
+        fa.h_scales = d_h_scales;
+        AH_HIP(ctx, hipSetDevice(ctx->device));
+        const int32_t qst = few_quantize(ctx, fa, stream, nullptr, 0);
+        if (qst) return qst;
+        AH_HIP(ctx, ah_launch_few(t, fa, true, pick(ctx, stream)));
+        return AH_OK;
     }
     // two passes: gate and up as one grouped GEMM (part order: up's refusals keyed after all of
     // gate's), then

@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(kThreads) quant_kernel(QuantArgs q) {
                                      (unsigned long long)tok * q.n_in);
         if (!valid) continue;
         const uint32_t lq = threadIdx.x & 3, k0 = 32 * b + 8 * lq;
-        int8_t *dst = q.codes + (size_t)tok * q.n_in + k0;
+        int8_t *dst = q.codes + (size_t)tok * q.pitch + k0;
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             if (k0 + k < q.n_in) dst[k] = (int8_t)(((k < 4 ? o.c0 : o.c1) >> (8 * (k & 3))) & 0xffu);

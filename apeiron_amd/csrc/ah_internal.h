@@ -333,9 +333,9 @@ constexpr unsigned long long kSeqTimeoutKey = 0ull;
 
 struct QuantArgs {
     const void *x;         // f32 or int64 [n_tok][n_in]
-    int8_t *codes;         // [n_tok][n_in]
+    int8_t *codes;         // n_tok rows of n_in, `pitch` bytes apart
     int64_t *scales;       // [n_tok][nb32]
-    uint32_t n_tok, n_in, nb32;
+    uint32_t n_tok, n_in, nb32, pitch;
     uint32_t src;          // AH_SRC_F32 / AH_SRC_Q32
     unsigned long long *status;
 };

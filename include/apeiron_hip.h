@@ -289,7 +289,7 @@ int32_t ah_seq_info(const ah_seq *seq, uint32_t *grid, uint32_t *act_bytes);
 
 /* y[n_tok][n_out] (token-major) = X W^T for X[n_tok][n_in] f32; quantization is a separate
  * in-stream pass into context scratch (grown on demand, never shrunk), which also holds split-K
- * partials.  GEMM calls on one context share that scratch: calls on different streams of the same
+ * partials.  (Calls of a few tokens quantize inside the kernel where that is cheaper.)  GEMM calls on one context share that scratch: calls on different streams of the same
  * context must not overlap (use one context per stream for concurrent prefills). */
 int32_t ah_gemm_f32_dev(ah_ctx *ctx, const ah_tensor *w, const float *d_x, size_t n_tok,
                         float *d_y, void *stream);
@@ -322,7 +322,8 @@ int32_t ah_gemm_q8_dev(ah_ctx *ctx, const ah_tensor *w, const int8_t *d_codes,
  *     min term, dmin m_j times the token's scaled code sum (two more bf16 outer products);
  *   AH_GEMM_DESIGN_F16: v_mfma_f32_32x32x16_f16 on exact f16 operands (the K-quants' design);
  *   AH_GEMM_DESIGN_AUTO (the default): the F16 design, measured 17-25% faster on MI355X at the
- *     configs[3] shapes (N = 512).
+ *     configs[3] shapes (N = 512); up to 32 tokens, where the activations fit a CU's LDS, a
+ *     one-launch kernel of its own (int8 block dots folded per block as the GEMV folds them).
  *   AH_GEMM_DESIGN_F16_TILE: the dequantize-once design for Q4_K, Q2_K and Q3_K: each 256-thread
  *     workgroup owns a 128-row x 128-token tile, converts each weight super-block to exact f16
  *     (sc * q, folded with d and the min term per super-block) once into LDS, and every wave

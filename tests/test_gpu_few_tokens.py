@@ -1,0 +1,140 @@
+"""GPU parity of the few-token GEMM (calls of at most 32 tokens) through the C ABI, at the sizes where
+it can go wrong: every family, one to 32 tokens around its 16-token operand tiles, widths off its
+16-row tiles, K around its units of 128 / 256 and its waves' K splits, rows too long for one tile's
+LDS (two token tiles, then the tile GEMM), f32 inputs quantized in the kernel and by a launch of
+their own, code rows off dword boundaries, payloads that end at their last byte, the SwiGLU epilogue
+of the prefill FFN, and a QuantAct scale whose products leave int64.
+
+Tolerance: every 32-block (or super-block half) is one exact integer dot folded with at most four
+f32 roundings, and the blocks' sums with one each, so an output is within (blocks + 8) * 2^-24 of the
+sum of its terms' magnitudes; the min terms are summed apart from the dots, which at most doubles
+that sum over sum|w * xhat| for these payloads.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from apeiron_amd import chart, synth
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+Q32 = 2.0 ** -32
+Q5_0, Q8_0, Q2_K, Q3_K, Q4_K, Q6_K = 6, 8, 10, 11, 12, 14
+ALL = [Q5_0, Q8_0, Q2_K, Q3_K, Q4_K, Q6_K]
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "GPU tests need the MI355X"
+    d = chart.Device(0)
+    yield d
+    d.close()
+
+
+def stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def payload(t, rng, n_out, n_in):
+    """Weights that average about zero, as trained ones do: no output is a near-cancellation."""
+    return synth.q4_k_centered_payload(rng, n_out, n_in) if t == Q4_K else synth.payload(t, rng, n_out, n_in)
+
+
+def close(t, raw, n_out, n_in, codes, scales, y, what):
+    for c in range(codes.shape[0]):
+        st, ref = oracle.matvec_q8act(t, raw, n_out, n_in, codes[c], scales[c])
+        st2, absdot = oracle.row_absdot(t, raw, n_out, n_in, codes[c], scales[c])
+        assert st == 0 and st2 == 0
+        err = np.abs(y[c].astype(np.float64) - ref.astype(np.float64) * Q32)
+        tol = 2 * (n_in / 32 + 8) * 2.0 ** -24 * absdot + Q32
+        bad = np.nonzero(~(err <= tol))[0]
+        assert bad.size == 0, f"{what} token {c}: rows {bad[:6]} err {err[bad[:6]]} tol {tol[bad[:6]]}"
+
+
+@pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("n_tok,n_out,n_in", [
+    (1, 16, 32), (2, 17, 256), (8, 130, 300), (9, 48, 901), (16, 33, 1536), (17, 40, 1000), (32, 129, 520),
+    (3, 20, 4864), (16, 18, 8960),   # waves of several units; two tiles of 8 tokens
+    (2, 16, 32768),                  # past the LDS: the tile GEMM
+])
+def test_few_tokens_vs_oracle(dev, t, n_tok, n_out, n_in):
+    rng = synth.rng_for(9, 1000 * t + n_in + n_tok)
+    raw = payload(t, rng, n_out, n_in)
+    x = synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)
+    st, codes, scales = oracle.quant_act_f32_batch(x)
+    assert st == 0
+    # the weight in a buffer that ends with its payload
+    dw = torch.from_numpy(raw).cuda()
+    for w in (dev.upload(t, raw, n_out, n_in), dev.wrap(t, dw.data_ptr(), raw.nbytes, n_out, n_in)):
+        y = torch.full((n_tok, n_out), float("nan"), device="cuda")
+        dx = torch.from_numpy(x).cuda()
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+        assert dev.sync_status(stream()) == 0
+        close(t, raw, n_out, n_in, codes, scales, y.cpu().numpy(), "f32")
+        # from codes, once at an odd address (rows off dword boundaries): the same outputs
+        for off in (0, 1):
+            dc = torch.zeros(n_tok * n_in + off, dtype=torch.int8, device="cuda")
+            dc[off:] = torch.from_numpy(codes.reshape(-1)).cuda()
+            ds = torch.from_numpy(scales).cuda()
+            yq = torch.full((n_tok, n_out), float("nan"), device="cuda")
+            w.gemm_q8_dev(dc.data_ptr() + off, ds.data_ptr(), n_tok, yq.data_ptr(), stream())
+            assert dev.sync_status(stream()) == 0
+            assert (yq == y).all(), (off, int((yq != y).sum()))
+        w.free()
+
+
+@pytest.mark.parametrize("gt,dt,n_embd,n_ff,n_tok", [
+    (Q4_K, Q6_K, 1536, 333, 8), (Q8_0, Q8_0, 256, 300, 1), (Q6_K, Q5_0, 512, 1000, 17), (Q5_0, Q2_K, 96, 64, 5),
+    (Q3_K, Q3_K, 901, 130, 16), (Q2_K, Q4_K, 1536, 96, 31), (Q8_0, Q4_K, 2048, 100, 6),  # (the last: six K splits, two passes)
+])
+def test_few_tokens_ffn(dev, gt, dt, n_embd, n_ff, n_tok):
+    """The SwiGLU epilogue: gate / up equal the projections' own calls, the hidden QuantAct is the
+    oracle's of those values, and down is the projection of it."""
+    rng = synth.rng_for(10, gt * 100 + n_ff)
+    raws = [payload(t, rng, o, i) for t, o, i in ((gt, n_ff, n_embd), (gt, n_ff, n_embd), (dt, n_embd, n_ff))]
+    G, U, D = (dev.upload(t, r, o, i) for r, (t, o, i) in zip(raws, ((gt, n_ff, n_embd), (gt, n_ff, n_embd), (dt, n_embd, n_ff))))
+    x = (synth.activations(rng, n_embd, n_tok).reshape(n_tok, n_embd) * np.float32(2.0 ** -6))
+    dx = torch.from_numpy(x).cuda()
+    gy, uy, g1, u1 = (torch.full((n_tok, n_ff), float("nan"), device="cuda") for _ in range(4))
+    hc = torch.zeros((n_tok, n_ff), dtype=torch.int8, device="cuda")
+    hs = torch.zeros((n_tok, -(-n_ff // 32)), dtype=torch.int64, device="cuda")
+    chart.ffn_gate_up_prefill_dev(dev, G, U, dx.data_ptr(), n_tok, hc.data_ptr(), hs.data_ptr(), gy.data_ptr(), uy.data_ptr(), stream())
+    chart.gemm_group_f32_dev(dev, [G, U], dx.data_ptr(), n_tok, [g1.data_ptr(), u1.data_ptr()], stream())
+    assert dev.sync_status(stream()) == 0
+    assert (gy == g1).all() and (uy == u1).all()
+    st, codes, scales = oracle.quant_act_f32_batch(x)
+    close(gt, raws[0], n_ff, n_embd, codes, scales, gy.cpu().numpy(), "gate")
+    HC, HS, g, u = hc.cpu().numpy(), hs.cpu().numpy(), gy.cpu().numpy(), uy.cpu().numpy()
+    for t in range(n_tok):
+        st, c, s, _ = oracle.swiglu_quant_f32(g[t], u[t])
+        assert st == 0 and (HC[t] == c).all() and (HS[t] == s).all(), t
+    y = torch.full((n_tok, n_embd), float("nan"), device="cuda")
+    hc2, hs2 = torch.zeros_like(hc), torch.zeros_like(hs)
+    chart.ffn_prefill_dev(dev, G, U, D, dx.data_ptr(), n_tok, y.data_ptr(), hc2.data_ptr(), hs2.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0
+    assert (hc2 == hc).all() and (hs2 == hs).all()
+    close(dt, raws[2], n_embd, n_ff, HC, HS, y.cpu().numpy(), "down")
+    for w in (G, U, D):
+        w.free()
+
+
+@pytest.mark.parametrize("n_in", [256, 8960])
+def test_few_tokens_refusals(dev, n_in):
+    """Input refusals recorded by the in-kernel quantizer, the separate one (the longer rows) and the
+    codes' own check, each the contract's first."""
+    n_tok, n_out = 9, 32
+    rng = synth.rng_for(11, n_in)
+    raw = payload(Q4_K, rng, n_out, n_in)
+    w = dev.upload(Q4_K, raw, n_out, n_in)
+    y = torch.zeros((n_tok, n_out), device="cuda")
+    x = synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)
+    st, codes, scales = oracle.quant_act_f32_batch(x)
+    x[7, 3], x[5, n_in - 1] = np.float32("nan"), np.float32(2.0 ** 40)
+    w.gemm_f32_dev(torch.from_numpy(x).cuda().data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 11  # token 5's range before token 7's NaN
+    scales[6, -1] = 1 << 62
+    codes[6, n_in - 32:] = 5
+    w.gemm_q8_dev(torch.from_numpy(codes).cuda().data_ptr(), torch.from_numpy(scales).cuda().data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 7
+    w.free()

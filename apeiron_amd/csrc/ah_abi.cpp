@@ -494,13 +494,29 @@ int32_t reset_status(ah_ctx *ctx) {
 // Its tokens per workgroup (all of them up to 32, as far as their quantized rows fit a CU's LDS); 0:
 // the call takes the tile GEMM.  At most two token tiles: each streams the weights again, and from
 // the third on the tile GEMM is faster (Q4_K 1536 x 8960 from codes, tiles of 8 tokens: 14.3 us
-// against 24.1 at 16 tokens, 24.9 against 20.1 at 24).  Past 16 tokens a family with min terms takes
-// the tile GEMM once its rows fill the device (from f32, 32 tokens: Q4_K 8960 x 1536 19.6 us against
-// 17.7, 896 x 896 13.1 against 15.2; Q8_0 8960 x 1536 17.9 against 26.1).
+// against 24.1 at 16 tokens, 24.9 against 20.1 at 24).
+// Past 16 tokens a workgroup takes all of them where two tiles of 16 would not fit the CUs together,
+// else the two tiles side by side (few_tile_of_run; both forms' outputs are the same bits): in
+// two tiles 24 tokens of Q4_K 2500 x 3000 from f32 take 15.2 us against 20.2 in one (the tile GEMM
+// 17.9) and a Q4_K / Q6_K q/k/v at 1536 23.0 against 32.4 (26.0); 17 tokens of Q8_0 8960 x 1536 in
+// one tile 12.7 against 17.5 in two (26.2).
+// A family with min terms, whose tile GEMM is the fastest, keeps it past 16 tokens where they do not
+// fit: Q4_K 8960 x 1536 from f32 at 32 tokens 19.6 us against 17.7.
 constexpr size_t kFewTokens = 32;
+uint32_t few_waves(uint32_t splits) { return splits >= 8 ? splits : 8 / splits * splits; }
+// Workgroups of one token tile.
+size_t few_wgs(uint32_t type, size_t n_out, size_t n_in) {
+    const uint32_t s = ah_few_splits(type, (uint32_t)n_in), rows = 16 * (few_waves(s) / s);
+    return (n_out + rows - 1) / rows;
+}
+uint32_t few_tile_of_run(const ah_ctx *ctx, uint32_t tile, size_t wgs) {
+    return tile == 32 && 2 * wgs <= (size_t)ctx->cu_count ? 16u : tile;
+}
 uint32_t few_tok_tile(const ah_ctx *ctx, const ah_tensor *t, size_t n_tok) {
     if (n_tok > kFewTokens || ctx->design[t->type] != AH_GEMM_DESIGN_AUTO) return 0;
-    if (n_tok > 16 && (t->type == AH_GGML_Q4_K || t->type == AH_GGML_Q2_K) && t->n_out > 16 * (size_t)ctx->cu_count) return 0;
+    if (n_tok > 16 && (t->type == AH_GGML_Q4_K || t->type == AH_GGML_Q2_K) &&
+        2 * few_wgs(t->type, t->n_out, t->n_in) > (size_t)ctx->cu_count)
+        return 0;
     uint32_t tok = n_tok > 16 ? 32u : 16u;
     while (tok >= 8 && ah_few_lds_bytes(t->type, kpad_of(t->n_in), n_tok < tok ? (uint32_t)n_tok : tok, kFewMaxWaves) > 160 * 1024)
         tok /= 2;
@@ -666,12 +682,15 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
             const uint32_t type = w[i]->type;
             FewArgs fa = few_args(src, x, scales_in, (uint32_t)n_in_sz, (uint32_t)n_tok, tile, status);
             fa.splits = ah_few_splits(type, fa.n_in);
-            fa.waves = fa.splits >= 8 ? fa.splits : 8 / fa.splits * fa.splits;
+            fa.waves = few_waves(fa.splits);
+            size_t wgs = 0;
             for (; i < n_parts && fa.n_parts < kFewMaxParts; ++i) {
                 if (w[i]->n_out == 0) continue;
                 if (w[i]->type != type || few(w[i]) != tile) break;
                 fa.p[fa.n_parts++] = few_part(w[i], y[i], key0[i]);
+                wgs += few_wgs(type, w[i]->n_out, fa.n_in);
             }
+            fa.tok_tile = few_tile_of_run(ctx, tile, wgs);
             if (q.x) {
                 fa.x = q.x;
                 fa.scales = q.scales;
@@ -1329,6 +1348,7 @@ static int32_t ffn_prefill_gate_up(ah_ctx *ctx, const ah_tensor *gate, const ah_
         fa.p[1] = few_part(up, nullptr, 0);
         fa.splits = ffn_splits;
         fa.waves = 4 * fa.splits;
+        fa.tok_tile = few_tile_of_run(ctx, tile, (n_ff + 31) / 32);
         fa.gy = d_gate_y;
         fa.uy = d_up_y;
         fa.h_codes = d_h_codes;

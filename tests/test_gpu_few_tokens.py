@@ -86,7 +86,8 @@ def test_few_tokens_vs_oracle(dev, t, n_tok, n_out, n_in):
 
 @pytest.mark.parametrize("gt,dt,n_embd,n_ff,n_tok", [
     (Q4_K, Q6_K, 1536, 333, 8), (Q8_0, Q8_0, 256, 300, 1), (Q6_K, Q5_0, 512, 1000, 17), (Q5_0, Q2_K, 96, 64, 5),
-    (Q3_K, Q3_K, 901, 130, 16), (Q2_K, Q4_K, 1536, 96, 31), (Q8_0, Q4_K, 2048, 100, 6),  # (the last: six K splits, two passes)
+    (Q3_K, Q3_K, 901, 130, 16), (Q2_K, Q4_K, 1536, 96, 31),
+    (Q4_K, Q4_K, 300, 4200, 19), (Q8_0, Q4_K, 2048, 100, 6),  # (the last: six K splits, two passes)
 ])
 def test_few_tokens_ffn(dev, gt, dt, n_embd, n_ff, n_tok):
     """The SwiGLU epilogue: gate / up equal the projections' own calls, the hidden QuantAct is the
@@ -117,6 +118,30 @@ def test_few_tokens_ffn(dev, gt, dt, n_embd, n_ff, n_tok):
     close(dt, raws[2], n_embd, n_ff, HC, HS, y.cpu().numpy(), "down")
     for w in (G, U, D):
         w.free()
+
+
+@pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("n_tok", [17, 25, 32])
+def test_one_token_tile_of_32_and_two_of_16_agree(dev, t, n_tok):
+    """Past 16 tokens the tokens of a workgroup follow the run's size: the parts alone take two tiles of
+    16, side by side in a group they fill the CUs and take one of 32.  The same bits, and the oracle's."""
+    n_in, n_out = 520, 4200
+    rng = synth.rng_for(12, 100 * t + n_tok)
+    raws = [payload(t, rng, n_out, n_in) for _ in range(4)]
+    ws = [dev.upload(t, raw, n_out, n_in) for raw in raws]
+    x = synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)
+    st, codes, scales = oracle.quant_act_f32_batch(x)
+    assert st == 0
+    dx = torch.from_numpy(x).cuda()
+    ys, y1 = ([torch.full((n_tok, n_out), float("nan"), device="cuda") for _ in ws] for _ in range(2))
+    chart.gemm_group_f32_dev(dev, ws, dx.data_ptr(), n_tok, [y.data_ptr() for y in ys], stream())
+    for w, y in zip(ws, y1):
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0
+    for w, y, one in zip(ws, ys, y1):
+        assert torch.equal(y, one)
+        w.free()
+    close(t, raws[0], n_out, n_in, codes, scales, ys[0].cpu().numpy(), "group")
 
 
 @pytest.mark.parametrize("n_in", [256, 8960])

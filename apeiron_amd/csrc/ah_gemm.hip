@@ -95,9 +95,44 @@ struct GemmPartArgs {
     uint32_t stages_per_split; // K stages of 64 per split (multiple of the kernel's unroll)
     uint32_t splits, wg_begin;
     uint32_t tok_tiles;        // token tiles of the part's type
+    uint32_t tok_chunk;        // token tiles per chunk (tile_of): tok_tiles where one chunk holds them all
+    uint32_t row_splits;       // row tiles x splits
     uint32_t type;             // GGUF type (read by the mixed K-quant kernel)
     uint64_t key0;             // added to the part's output refusal keys (GemmPartDesc::key0)
 };
+// The tile of a part's logical workgroup Lp: chunk of token tiles, then row tile, split, and token
+// tile of the chunk fastest.  Workgroups that run together on an XCD then read one weight tile and
+// one chunk of the operand, which stays in that XCD's 4 MB L2 while every row tile passes over it.
+// In one chunk, 2048 tokens x 1536 columns are 6 MB and each row tile reads them from the Infinity
+// Cache again.  See chunk_tiles for the measured sizes.
+struct TileId {
+    uint32_t tt, split, rtile;
+};
+template <bool CHUNK = true>
+AH_DEV TileId tile_of(const GemmPartArgs &pa, uint32_t Lp) {
+    if constexpr (!CHUNK) {
+        const uint32_t rest = Lp / pa.tok_tiles;
+        return {Lp % pa.tok_tiles, rest % pa.splits, rest / pa.splits};
+    }
+    const uint32_t t0 = Lp / (pa.tok_chunk * pa.row_splits) * pa.tok_chunk;
+    const uint32_t tw = pa.tok_tiles - t0 < pa.tok_chunk ? pa.tok_tiles - t0 : pa.tok_chunk;
+    const uint32_t Lc = Lp - t0 * pa.row_splits, rest = Lc / tw;
+    return {t0 + Lc % tw, rest % pa.splits, rest / pa.splits};
+}
+// Token tiles per chunk: equal chunks of at most kChunkBytes of operand columns of one split (half of
+// an XCD's L2; the rest is for the weights and the outputs passing through).  us at 2048 tokens in
+// one chunk, then in chunks of 3, 2, 1 and 0.5 MB: Q4_K 17920x1536 224, 205, 195, 193, 205; Q4_K
+// 1536x8960 127, 124, 118, 118, 119; Q8_0 17920x1536 272, 261, 257, 269, 261; Q6_K 1536x8960 202,
+// 187, 189, 194, 196; the tile design's Q3_K 17920x1536 263 in one, 247 in 2 MB.  At 512 tokens of
+// 8960 columns (two or three chunks) the differences are within the noise: Q4_K 47.2 and 45.2, Q6_K
+// 68.1 and 67.4.
+constexpr uint64_t kChunkBytes = 2u << 20;
+inline uint32_t chunk_tiles(uint32_t tok_tiles, uint32_t tok, uint32_t k) {
+    const uint64_t fit = kChunkBytes / ((uint64_t)tok * k * 2u);
+    if (fit >= tok_tiles) return tok_tiles;
+    const uint32_t most = fit ? (uint32_t)fit : 1u, chunks = (tok_tiles + most - 1) / most;
+    return (tok_tiles + chunks - 1) / chunks;
+}
 struct GemmArgs {
     GemmPartArgs p[kGemmMaxParts];
     uint32_t n_parts, n_in, n_tok, kpad;
@@ -607,7 +642,7 @@ AH_DEV __attribute__((always_inline)) void gemm_store(const GemmArgs &a, const G
 }
 
 // The kernel body, on an LDS ring of RG slots of buf_bytes<TYPE> at `lds`.
-template <int TYPE, int WV, int RG>
+template <int TYPE, int WV, int RG, bool CHUNK = true>
 // (by value: with a reference to the kernel argument the Q8_0 kernel grows from 207 to 256 VGPRs)
 AH_DEV __attribute__((always_inline)) void gemm_rb_body(GemmArgs a, uint8_t *lds_base) {
     constexpr int NN = rb::kNN, NM = rb::nm<TYPE>(), NW = rb::nw<TYPE, RG>(), DW = rb::dw<TYPE, RG>();
@@ -633,8 +668,8 @@ AH_DEV __attribute__((always_inline)) void gemm_rb_body(GemmArgs a, uint8_t *lds
         if (i < a.n_parts && L >= a.p[i].wg_begin) pi = i;
     const GemmPartArgs &pa = a.p[pi];
     const uint32_t Lp = L - pa.wg_begin;
-    const uint32_t tt = Lp % pa.tok_tiles, rest = Lp / pa.tok_tiles;
-    const uint32_t split = rest % pa.splits, rtile = rest / pa.splits;
+    const TileId id = tile_of<CHUNK>(pa, Lp);
+    const uint32_t tt = id.tt, split = id.split, rtile = id.rtile;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = lane & 31, h = lane >> 5;
@@ -950,10 +985,13 @@ AH_DEV __attribute__((always_inline)) void gemm_rb_body(GemmArgs a, uint8_t *lds
                              rb::lds_bytes<TYPE, WV, RG>());
 }
 
-template <int TYPE, int WV, int RG>
+// CHUNK false: every part's token tiles are one chunk.  Q4_K holds both forms: its kernel has 128
+// VGPRs and no scalar register to spare, and the chunk arithmetic's spills cost 2 us of a call of one
+// chunk (8960x1536, 24 tokens: 18.5 us without, 20.0 with); the other kernels take it at no cost.
+template <int TYPE, int WV, int RG, bool CHUNK = TYPE != AH_GGML_Q4_K>
 __global__ void __launch_bounds__(64 * WV, TYPE == AH_GGML_Q4_K ? 4 : 2) gemm_rb_kernel(GemmArgs a) {
     __shared__ __align__(16) uint8_t lds[rb::lds_bytes<TYPE, WV, RG>()];
-    gemm_rb_body<TYPE, WV, RG>(a, lds);
+    gemm_rb_body<TYPE, WV, RG, CHUNK>(a, lds);
 }
 
 // ---- int8-MFMA design (Q8_0; Q4_K below) ------------------------------------------------------
@@ -1687,8 +1725,8 @@ __global__ void __launch_bounds__(256, 2) gemm_dq_kernel(GemmArgs a) {
         if (i < a.n_parts && L >= a.p[i].wg_begin) pi = i;
     const GemmPartArgs &pa = a.p[pi];
     const uint32_t Lp = L - pa.wg_begin;
-    const uint32_t tt = Lp % pa.tok_tiles, rest = Lp / pa.tok_tiles;
-    const uint32_t split = rest % pa.splits, rtile = rest / pa.splits;
+    const TileId id = tile_of(pa, Lp);
+    const uint32_t tt = id.tt, split = id.split, rtile = id.rtile;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, j = lane & 31u, h = lane >> 5;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2085,6 +2123,7 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
     a.xsx = xsx;
     a.ffn = ffn_form ? *ffn : GemmFfn{};
     uint32_t wg = 0;
+    bool chunked = false;
     for (uint32_t i = 0; i < kGemmMaxParts; ++i) {
         GemmPartArgs &P = a.p[i];
         if (i >= n_parts) {
@@ -2110,7 +2149,10 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
         P.type = pt;
         P.key0 = d.key0;
         const uint32_t rows = ffn_form ? g.rows / 2 : g.rows;  // FFN: a tile's rows are hidden pairs
-        wg += ((d.n_out + rows - 1) / rows) * P.tok_tiles * P.splits;
+        P.row_splits = ((d.n_out + rows - 1) / rows) * P.splits;
+        P.tok_chunk = chunk_tiles(P.tok_tiles, g.toks, kpad / P.splits);
+        chunked = chunked || P.tok_chunk != P.tok_tiles;
+        wg += P.row_splits * P.tok_tiles;
     }
     a.n_wg = wg;
     if (wg == 0) return hipSuccess;
@@ -2146,7 +2188,10 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
     case kGemmMixedKQuant: hipLaunchKernelGGL(gemm_rb_kquant_kernel, rb_grid, blk, 0, stream, a); break;
     case AH_GGML_Q8_0: AH_GFORMS(AH_GGML_Q8_0) break;
     case AH_GGML_Q5_0: AH_GFORMS(AH_GGML_Q5_0) break;
-    case AH_GGML_Q4_K: hipLaunchKernelGGL((gemm_rb_kernel<AH_GGML_Q4_K, 4, 4>), rb_grid, blk, 0, stream, a); break;
+    case AH_GGML_Q4_K:
+        if (chunked) hipLaunchKernelGGL((gemm_rb_kernel<AH_GGML_Q4_K, 4, 4, true>), rb_grid, blk, 0, stream, a);
+        else hipLaunchKernelGGL((gemm_rb_kernel<AH_GGML_Q4_K, 4, 4>), rb_grid, blk, 0, stream, a);
+        break;
     case AH_GGML_Q6_K: AH_GFORMS(AH_GGML_Q6_K) break;
     default: return hipErrorInvalidValue;
     }

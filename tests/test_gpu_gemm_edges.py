@@ -485,3 +485,43 @@ def test_k23_refusal_order_across_tokens(dev, t, design):
     finally:
         dev.set_gemm_design(t, 0)
         w.free()
+
+
+# ---- the order of token tiles: chunks ------------------------------------------------------
+# The grid walks the token tiles in chunks whose operand columns fit 2 MB: here two to four chunks
+# of unequal sizes, the last tile ragged, one row tile ragged, with K splits and without, and one
+# chunk exactly.  The tokens repeat 64 distinct ones in an order that differs from tile to tile: a
+# token's output does not depend on its tile, so equal tokens have bit-equal outputs, and the
+# distinct ones are held to the oracle with this file's bar.
+@pytest.mark.parametrize("t,n_out,n_in,n_tok,form", [
+    (12, 700, 8960, 1337, 0), (12, 33, 32768, 999, 0), (8, 300, 8960, 1409, 0), (6, 130, 16384, 1100, 0),
+    (14, 300, 8960, 1793, 0), (12, 300, 8960, 640, 0), (12, 160, 16384, 1337, 3), (11, 160, 16384, 999, 0),
+    (10, 130, 16384, 700, 0),
+])
+def test_token_tile_chunks(dev, t, n_out, n_in, n_tok, form):
+    rng = synth.rng_for(11, 100 * t + n_tok)
+    raw = synth.q4_k_centered_payload(rng, n_out, n_in) if t == 12 else synth.payload(t, rng, n_out, n_in)
+    base = synth.activations(rng, n_in, 64).reshape(64, n_in)
+    st, codes, scales = oracle.quant_act_f32_batch(base)
+    assert st == 0
+    i = np.arange(n_tok)
+    order = (37 * i + i // 64) % 64
+    w = dev.upload(t, raw, n_out, n_in)
+    y = torch.full((n_tok, n_out), float("nan"), device="cuda")
+    dx = to_dev(base[order])
+    dev.set_gemm_design(t, form)
+    try:
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+        assert dev.sync_status(stream()) == 0
+    finally:
+        dev.set_gemm_design(t, 0)
+    y = y.cpu().numpy()
+    for c in range(64):
+        same = y[order == c]
+        assert (same.view(np.int32) == same[0].view(np.int32)).all(), c
+        st, ref = oracle.matvec_q8act(t, raw, n_out, n_in, codes[c], scales[c])
+        st2, absdot = oracle.row_absdot(t, raw, n_out, n_in, codes[c], scales[c])
+        assert st == 0 and st2 == 0
+        err = np.abs(same[0].astype(np.float64) - ref.astype(np.float64) * Q32)
+        assert (err <= TOL * absdot + Q32).all(), (c, err.max())
+    w.free()

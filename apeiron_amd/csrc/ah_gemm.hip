@@ -110,7 +110,7 @@ struct TileId {
 };
 template <bool CHUNK = true>
 AH_DEV TileId tile_of(const GemmPartArgs &pa, uint32_t Lp) {
-    if constexpr (!CHUNK) {
+    if (!CHUNK || pa.tok_chunk == pa.tok_tiles) {
         const uint32_t rest = Lp / pa.tok_tiles;
         return {Lp % pa.tok_tiles, rest % pa.splits, rest / pa.splits};
     }
@@ -123,13 +123,16 @@ AH_DEV TileId tile_of(const GemmPartArgs &pa, uint32_t Lp) {
 // an XCD's L2; the rest is for the weights and the outputs passing through).  us at 2048 tokens in
 // one chunk, then in chunks of 3, 2, 1 and 0.5 MB: Q4_K 17920x1536 224, 205, 195, 193, 205; Q4_K
 // 1536x8960 127, 124, 118, 118, 119; Q8_0 17920x1536 272, 261, 257, 269, 261; Q6_K 1536x8960 202,
-// 187, 189, 194, 196; the tile design's Q3_K 17920x1536 263 in one, 247 in 2 MB.  At 512 tokens of
-// 8960 columns (two or three chunks) the differences are within the noise: Q4_K 47.2 and 45.2, Q6_K
-// 68.1 and 67.4.
-constexpr uint64_t kChunkBytes = 2u << 20;
-inline uint32_t chunk_tiles(uint32_t tok_tiles, uint32_t tok, uint32_t k) {
-    const uint64_t fit = kChunkBytes / ((uint64_t)tok * k * 2u);
-    if (fit >= tok_tiles) return tok_tiles;
+// 187, 189, 194, 196; the tile design's Q3_K 17920x1536 263 in one, 247 in 2 MB.
+// One chunk where the row tiles read the operand for less than kChunkReads bytes in all: there are
+// then few of them to an XCD, and the time is the K loop's.  2048 tokens, one chunk and 2 MB: Q8_0
+// 512x8960 (147 MB) 81.3 and 72.3, 1280x1536 (63 MB) 44.1 and 44.6.  Q4_K's chunked kernel costs 2 us
+// more (gemm_rb_kernel), so its line is higher: 768x8960 (220 MB) 79.2 and 79.5, 1280x8960 (367 MB)
+// 116.0 and 112.9.
+constexpr uint64_t kChunkBytes = 2u << 20, kChunkReads = 96u << 20, kChunkReadsQ4K = 256u << 20;
+inline uint32_t chunk_tiles(uint32_t type, uint32_t row_tiles, uint32_t tok_tiles, uint32_t tok, uint32_t kpad, uint32_t splits) {
+    const uint64_t tile = (uint64_t)tok * kpad * 2u, fit = kChunkBytes * splits / tile;
+    if (fit >= tok_tiles || tile * tok_tiles * row_tiles < (type == AH_GGML_Q4_K ? kChunkReadsQ4K : kChunkReads)) return tok_tiles;
     const uint32_t most = fit ? (uint32_t)fit : 1u, chunks = (tok_tiles + most - 1) / most;
     return (tok_tiles + chunks - 1) / chunks;
 }
@@ -985,10 +988,10 @@ AH_DEV __attribute__((always_inline)) void gemm_rb_body(GemmArgs a, uint8_t *lds
                              rb::lds_bytes<TYPE, WV, RG>());
 }
 
-// CHUNK false: every part's token tiles are one chunk.  Q4_K holds both forms: its kernel has 128
-// VGPRs and no scalar register to spare, and the chunk arithmetic's spills cost 2 us of a call of one
-// chunk (8960x1536, 24 tokens: 18.5 us without, 20.0 with); the other kernels take it at no cost.
-template <int TYPE, int WV, int RG, bool CHUNK = TYPE != AH_GGML_Q4_K>
+// CHUNK false: every part's token tiles are one chunk.  The chunk arithmetic costs a call of one
+// chunk 0.1 to 0.3 us, and Q4_K's kernel, with 128 VGPRs and no scalar register to spare, 2 us in
+// spills (8960x1536, 24 tokens: 18.5 us without, 20.0 with).
+template <int TYPE, int WV, int RG, bool CHUNK>
 __global__ void __launch_bounds__(64 * WV, TYPE == AH_GGML_Q4_K ? 4 : 2) gemm_rb_kernel(GemmArgs a) {
     __shared__ __align__(16) uint8_t lds[rb::lds_bytes<TYPE, WV, RG>()];
     gemm_rb_body<TYPE, WV, RG, CHUNK>(a, lds);
@@ -2149,8 +2152,9 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
         P.type = pt;
         P.key0 = d.key0;
         const uint32_t rows = ffn_form ? g.rows / 2 : g.rows;  // FFN: a tile's rows are hidden pairs
-        P.row_splits = ((d.n_out + rows - 1) / rows) * P.splits;
-        P.tok_chunk = chunk_tiles(P.tok_tiles, g.toks, kpad / P.splits);
+        const uint32_t row_tiles = (d.n_out + rows - 1) / rows;
+        P.row_splits = row_tiles * P.splits;
+        P.tok_chunk = chunk_tiles(pt, row_tiles, P.tok_tiles, g.toks, kpad, P.splits);
         chunked = chunked || P.tok_chunk != P.tok_tiles;
         wg += P.row_splits * P.tok_tiles;
     }
@@ -2158,10 +2162,11 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
     if (wg == 0) return hipSuccess;
     const dim3 rb_grid((a.n_wg + 7) / 8 * 8);
     const dim3 blk(64 * waves);
+#define AH_GFORM(T, W, R)                                                                               \
+    if (chunked) hipLaunchKernelGGL((gemm_rb_kernel<T, W, R, true>), rb_grid, blk, 0, stream, a);       \
+    else hipLaunchKernelGGL((gemm_rb_kernel<T, W, R, false>), rb_grid, blk, 0, stream, a);
 #define AH_GFORMS(T)                                                                                    \
-    if (form == kForm2x2) hipLaunchKernelGGL((gemm_rb_kernel<T, 2, 2>), rb_grid, blk, 0, stream, a);    \
-    else if (form == kForm2x4) hipLaunchKernelGGL((gemm_rb_kernel<T, 2, 4>), rb_grid, blk, 0, stream, a); \
-    else hipLaunchKernelGGL((gemm_rb_kernel<T, 4, 4>), rb_grid, blk, 0, stream, a);
+    if (form == kForm2x2) { AH_GFORM(T, 2, 2) } else if (form == kForm2x4) { AH_GFORM(T, 2, 4) } else { AH_GFORM(T, 4, 4) }
     if (ffn_form) {
         if (type == AH_GGML_Q4_K) hipLaunchKernelGGL((gemm_dq_kernel<AH_GGML_Q4_K, true>), rb_grid, dim3(256), 0, stream, a);
         else if (type == AH_GGML_Q2_K) hipLaunchKernelGGL((gemm_dq_kernel<AH_GGML_Q2_K, true>), rb_grid, dim3(256), 0, stream, a);
@@ -2188,14 +2193,12 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
     case kGemmMixedKQuant: hipLaunchKernelGGL(gemm_rb_kquant_kernel, rb_grid, blk, 0, stream, a); break;
     case AH_GGML_Q8_0: AH_GFORMS(AH_GGML_Q8_0) break;
     case AH_GGML_Q5_0: AH_GFORMS(AH_GGML_Q5_0) break;
-    case AH_GGML_Q4_K:
-        if (chunked) hipLaunchKernelGGL((gemm_rb_kernel<AH_GGML_Q4_K, 4, 4, true>), rb_grid, blk, 0, stream, a);
-        else hipLaunchKernelGGL((gemm_rb_kernel<AH_GGML_Q4_K, 4, 4>), rb_grid, blk, 0, stream, a);
-        break;
+    case AH_GGML_Q4_K: AH_GFORM(AH_GGML_Q4_K, 4, 4) break;
     case AH_GGML_Q6_K: AH_GFORMS(AH_GGML_Q6_K) break;
     default: return hipErrorInvalidValue;
     }
 #undef AH_GFORMS
+#undef AH_GFORM
     return hipGetLastError();
 }
 

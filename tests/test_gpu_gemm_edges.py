@@ -494,9 +494,9 @@ def test_k23_refusal_order_across_tokens(dev, t, design):
 # token's output does not depend on its tile, so equal tokens have bit-equal outputs, and the
 # distinct ones are held to the oracle with this file's bar.
 @pytest.mark.parametrize("t,n_out,n_in,n_tok,form", [
-    (12, 700, 8960, 1337, 0), (12, 33, 32768, 999, 0), (8, 300, 8960, 1409, 0), (6, 130, 16384, 1100, 0),
-    (14, 300, 8960, 1793, 0), (12, 300, 8960, 640, 0), (12, 160, 16384, 1337, 3), (11, 160, 16384, 999, 0),
-    (10, 130, 16384, 700, 0),
+    (12, 1300, 8960, 1730, 0), (12, 520, 32768, 999, 0), (8, 700, 8960, 1409, 0), (6, 600, 16384, 900, 0),
+    (14, 520, 8960, 1793, 0), (12, 300, 8960, 640, 0), (12, 1400, 8960, 1730, 3), (11, 420, 16384, 999, 0),
+    (10, 400, 16384, 1020, 0),
 ])
 def test_token_tile_chunks(dev, t, n_out, n_in, n_tok, form):
     rng = synth.rng_for(11, 100 * t + n_tok)

@@ -86,8 +86,10 @@ AH_DEV QuadIn quad_load(const void *x, const int64_t *scales, uint32_t src, uint
     for (int i = 0; i < 16; ++i) in.w[i] = 0;
     if (src == AH_SRC_F32) {
         const uint32_t *xb = static_cast<const uint32_t *>(x) + row_off + k0;
-        if (in.take == 8 && (reinterpret_cast<uintptr_t>(xb) & 15) == 0) {
-            const u32x4 a = reinterpret_cast<const u32x4 *>(xb)[0], c = reinterpret_cast<const u32x4 *>(xb)[1];
+        if (in.take == 8) {
+            u32x4 a, c;  // (rows of a length off 4 are dword-aligned: enough for a 16-byte global load)
+            __builtin_memcpy(&a, xb, 16);
+            __builtin_memcpy(&c, xb + 4, 16);
             in.w[0] = a.x; in.w[1] = a.y; in.w[2] = a.z; in.w[3] = a.w;
             in.w[4] = c.x; in.w[5] = c.y; in.w[6] = c.z; in.w[7] = c.w;
         } else {
@@ -347,11 +349,6 @@ AH_DEV QuadOut quad_quant(const QuadIn &in, uint32_t src, uint32_t b, unsigned l
     o.e = e;
     o.fsc = e < 0 ? 0.0f : __builtin_ldexpf(1.0f, e - 32);
     return o;
-}
-
-AH_DEV QuadOut quant_quad(const void *x, uint32_t src, uint32_t n_in, size_t row_off, uint32_t b,
-                          bool valid, unsigned long long *status, unsigned long long key_base) {
-    return quad_quant(quad_load(x, nullptr, src, n_in, row_off, b, valid), src, b, status, key_base);
 }
 
 // Store one quad's block to the LDS activation.

@@ -160,6 +160,32 @@ def test_quant_act_f32_refusals(dev):
     assert quant_f32_gpu(dev, np.ones((1, 64), np.float32))[0] == 0  # status was cleared
 
 
+@pytest.mark.parametrize("n_tok,n_in,off", [
+    (1, 1, 0), (2, 7, 1), (3, 8, 3), (130, 9, 1), (5, 31, 0), (5, 63, 2), (16, 40, 1), (7, 901, 3), (2048, 33, 1),
+    (66001, 32, 0), (2, 16777300, 1),  # more blocks than a workgroup's, then than one grid pass
+])
+def test_quant_act_f32_rows_at_any_alignment(dev, n_tok, n_in, off):
+    """Codes, scales and the bytes around them with rows, input and output at every dword / byte
+    offset: 16-byte loads and 8-byte stores only where a lane has 8 elements."""
+    rng = np.random.default_rng(n_in)
+    x = rng.standard_normal((n_tok, n_in)).astype(np.float32)
+    nb, size = -(-n_in // 32), n_tok * n_in
+    dx = torch.full((off + size,), float("nan"), dtype=torch.float32, device="cuda")
+    dx[off:] = to_dev(x.reshape(-1))
+    dc = torch.full((off + size + 9,), 99, dtype=torch.int8, device="cuda")
+    ds = torch.full((n_tok * nb + 1,), -5, dtype=torch.int64, device="cuda")
+    dev.quant_act_f32_dev(ptr(dx) + 4 * off, n_tok, n_in, ptr(dc) + off, ptr(ds), stream())
+    assert dev.sync_status(stream()) == 0
+    c, s = dc.cpu().numpy(), ds.cpu().numpy()
+    assert (c[:off] == 99).all() and (c[off + size:] == 99).all() and s[-1] == -5
+    pad = np.zeros((n_tok, 32 * nb), np.float32)
+    pad[:, :n_in] = x
+    st, oc, os_ = oracle.quant_act_f32(pad.reshape(-1))  # blocks are independent: zero padding codes 0
+    assert st == 0
+    assert (c[off:off + size].reshape(n_tok, n_in) == oc.reshape(n_tok, -1)[:, :n_in]).all()
+    assert (s[:-1] == os_).all()
+
+
 def test_quant_act_q32_reference_kats(dev):
     # chart/tests.rs:397-415
     q = dev.quant_act([3, 130, -3])

@@ -525,3 +525,26 @@ def test_token_tile_chunks(dev, t, n_out, n_in, n_tok, form):
         err = np.abs(same[0].astype(np.float64) - ref.astype(np.float64) * Q32)
         assert (err <= TOL * absdot + Q32).all(), (c, err.max())
     w.free()
+
+
+@pytest.mark.parametrize("n_in", [33, 901, 1537, 2049, 4866, 8957])
+@pytest.mark.parametrize("off", [0, 1, 6])
+def test_gemm_code_rows_at_any_byte(n_in, off):
+    """Code rows off the dword grid (n_in % 4 != 0, a base at any byte): the quantizer's codes give
+    the f32 input's outputs bit for bit, at every width class of the operand pass."""
+    d = chart.Device(0)
+    rng = np.random.default_rng(n_in + off)
+    n_tok, n_out = 40, 48
+    w = d.upload(8, synth.payload(8, rng, n_out, n_in), n_out, n_in)
+    s = torch.cuda.current_stream().cuda_stream
+    x = torch.from_numpy(rng.standard_normal((n_tok, n_in)).astype(np.float32)).cuda()
+    codes = torch.zeros(off + n_tok * n_in, dtype=torch.int8, device="cuda")
+    scales = torch.zeros(n_tok, -(-n_in // 32), dtype=torch.int64, device="cuda")
+    d.quant_act_f32_dev(x.data_ptr(), n_tok, n_in, codes.data_ptr() + off, scales.data_ptr(), s)
+    yc, yf = (torch.full((n_tok, n_out), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2))
+    w.gemm_q8_dev(codes.data_ptr() + off, scales.data_ptr(), n_tok, yc.data_ptr(), s)
+    w.gemm_f32_dev(x.data_ptr(), n_tok, yf.data_ptr(), s)
+    assert d.sync_status(s) == 0
+    assert torch.isfinite(yf).all() and torch.equal(yc, yf)
+    w.free()
+    d.close()

@@ -163,3 +163,26 @@ def test_few_tokens_refusals(dev, n_in):
     w.gemm_q8_dev(torch.from_numpy(codes).cuda().data_ptr(), torch.from_numpy(scales).cuda().data_ptr(), n_tok, y.data_ptr(), stream())
     assert dev.sync_status(stream()) == 7
     w.free()
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_K, Q2_K])  # (no code sums, a block's, a 16-group's)
+@pytest.mark.parametrize("n_in", [1, 15, 18, 31, 901, 1538, 4863])
+def test_few_tokens_code_rows_at_any_byte(dev, t, n_in):
+    """Code rows at every offset from the dword grid, other bytes around them, row ends inside and on a
+    16-code chunk: the f32 call's outputs, whose codes these are, bit for bit."""
+    n_out = 20
+    rng = synth.rng_for(13, 10 * n_in + t)
+    w = dev.upload(t, payload(t, rng, n_out, n_in), n_out, n_in)
+    for n_tok in (1, 3, 17):
+        dx = torch.from_numpy(synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)).cuda()
+        ds = torch.zeros((n_tok, -(-n_in // 32)), dtype=torch.int64, device="cuda")
+        y = torch.full((n_tok, n_out), float("nan"), device="cuda")
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+        for off in range(4):
+            dc = torch.full((off + n_tok * n_in + 7,), 77, dtype=torch.int8, device="cuda")
+            dev.quant_act_f32_dev(dx.data_ptr(), n_tok, n_in, dc.data_ptr() + off, ds.data_ptr(), stream())
+            yq = torch.full((n_tok, n_out), float("nan"), device="cuda")
+            w.gemm_q8_dev(dc.data_ptr() + off, ds.data_ptr(), n_tok, yq.data_ptr(), stream())
+            assert dev.sync_status(stream()) == 0
+            assert torch.equal(yq, y), (n_tok, off)
+    w.free()

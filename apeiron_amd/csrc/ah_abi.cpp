@@ -534,8 +534,6 @@ FewArgs few_args(uint32_t src, const void *x, const int64_t *scales, uint32_t n_
     a.kpad = kpad_of(n_in);
     a.src = src;
     a.pitch = n_in;
-    a.byte0 = src == AH_SRC_CODES ? (uint32_t)(reinterpret_cast<uintptr_t>(x) % 4) : 0u;
-    a.unaligned = src == AH_SRC_CODES && (n_in % 4 || a.byte0) ? 1u : 0u;
     a.tok_tile = tok_tile;
     return a;
 }

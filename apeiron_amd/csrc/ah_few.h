@@ -18,8 +18,6 @@ struct FewArgs {
     const int64_t *scales;    // [n_tok][ceil(n_in / 32)] with AH_SRC_CODES
     unsigned long long *status;
     uint32_t n_parts, n_in, n_tok, kpad, src, pitch;
-    uint32_t unaligned;       // codes rows do not start on dword boundaries
-    uint32_t byte0;           // codes: x's offset from the dword boundary below it
     uint32_t splits;          // waves along K of a row tile
     uint32_t waves;           // of a workgroup: splits x row tiles
     uint32_t tok_tile;        // tokens of a workgroup (<= 32)

@@ -99,15 +99,17 @@ AH_DEV void stage_f32(const FewArgs &a, const FewAct &A, uint32_t tok0, uint32_t
 // off the dword grid are read as the dwords that hold them, 16 bytes and one dword, and shifted: a
 // load a byte took 4861 x 901 of Q5_0 at 5 tokens 10.6 us (now 9.2), 1536 x 4865 of Q4_K at 16 tokens
 // 34.3 us (now 13.9).
-template <int TYPE>
+template <int TYPE, bool UNALIGNED>
 AH_DEV void stage_codes(const FewArgs &a, const FewAct &A, uint32_t tok0, uint32_t ntile) {
-    constexpr uint32_t kBatch = 4;
+    constexpr uint32_t kBatch = UNALIGNED ? 3 : 4;  // (4 would take the kernel past 80 VGPRs, a wave a SIMD less)
+    const uint32_t off = UNALIGNED ? (uint32_t)reinterpret_cast<uintptr_t>(a.x) & 3u : 0u;
     const uint32_t nch = a.kpad / 16, nb32 = (a.n_in + 31) / 32, total = ntile * nch;
-    const __amdgpu_buffer_rsrc_t rx = ah_rsrc(static_cast<const uint8_t *>(a.x) - a.byte0, a.n_tok * a.pitch + a.byte0), rsc = ah_rsrc(a.scales, a.n_tok * nb32 * 8u);
+    const __amdgpu_buffer_rsrc_t rx = ah_rsrc(static_cast<const uint8_t *>(a.x) - off, a.n_tok * a.pitch + off), rsc = ah_rsrc(a.scales, a.n_tok * nb32 * 8u);
     for (uint32_t base = 0; base < total; base += kBatch * blockDim.x) {
         u32x4 c[kBatch];
         u32x2 s[kBatch];
-        uint32_t tt[kBatch], kk[kBatch], past[kBatch];
+        uint32_t tt[kBatch], kk[kBatch];
+        [[maybe_unused]] uint32_t past[kBatch];
 #pragma unroll
         for (uint32_t j = 0; j < kBatch; ++j) {
             const uint32_t i = base + j * blockDim.x + threadIdx.x;
@@ -115,9 +117,9 @@ AH_DEV void stage_codes(const FewArgs &a, const FewAct &A, uint32_t tok0, uint32
             const bool in = i < total && k < a.n_in;
             tt[j] = t;
             kk[j] = k;
-            const uint32_t at = in ? ((tok0 + t) * a.pitch + k + a.byte0) & ~3u : kOob;
-            c[j] = ah_ld128(rx, at);
-            past[j] = a.unaligned ? ah_ld32(rx, in ? at + 16 : kOob) : 0u;
+            const uint32_t at = (tok0 + t) * a.pitch + k + off;
+            c[j] = ah_ld128(rx, in ? (UNALIGNED ? at & ~3u : at) : kOob);
+            if constexpr (UNALIGNED) past[j] = ah_ld32(rx, in ? (at & ~3u) + 16 : kOob);
             s[j] = ah_ld64(rsc, in ? 8 * ((tok0 + t) * nb32 + k / 32) : kOob);
         }
 #pragma unroll
@@ -125,8 +127,8 @@ AH_DEV void stage_codes(const FewArgs &a, const FewAct &A, uint32_t tok0, uint32
             const uint32_t i = base + j * blockDim.x + threadIdx.x, t = tt[j], k = kk[j];
             const uint32_t take = i < total && k < a.n_in ? (a.n_in - k < 16 ? a.n_in - k : 16) : 0;
             uint32_t w[4] = {c[j].x, c[j].y, c[j].z, c[j].w};
-            if (a.unaligned) {
-                const uint32_t sh = ((tok0 + t) * a.pitch + k + a.byte0) & 3u;
+            if constexpr (UNALIGNED) {
+                const uint32_t sh = ((tok0 + t) * a.pitch + k + off) & 3u;
                 w[0] = ah_alignbyte(w[1], w[0], sh);
                 w[1] = ah_alignbyte(w[2], w[1], sh);
                 w[2] = ah_alignbyte(w[3], w[2], sh);
@@ -445,7 +447,8 @@ __global__ void __launch_bounds__(64 * kFewMaxWaves) gemm_few_kernel(FewArgs a) 
     }
     if (u0 < W.u1) W.load(u0);
     if (a.src == AH_SRC_F32) stage_f32<TYPE>(a, A, tok0, ntile);
-    else stage_codes<TYPE>(a, A, tok0, ntile);
+    else if (((uint32_t)reinterpret_cast<uintptr_t>(a.x) | a.pitch) & 3u) stage_codes<TYPE, true>(a, A, tok0, ntile);
+    else stage_codes<TYPE, false>(a, A, tok0, ntile);
     ah_lds_barrier();
     for (uint32_t u = u0; u < W.u1; ++u) {
         W.stage(slot, lane);

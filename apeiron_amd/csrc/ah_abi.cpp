@@ -48,8 +48,8 @@ hipError_t ah_launch_gemm(uint32_t type, uint32_t n_parts, const GemmPartDesc *p
                           const GemmFfn *ffn = nullptr);
 hipError_t ah_launch_splitk_reduce(uint32_t n_parts, const GemmPartDesc *parts, uint32_t n_tok,
                                    const float *tok_scale, unsigned long long *status, hipStream_t stream);
-uint32_t ah_gemm_pick_splits(uint32_t type, uint32_t n_out, uint32_t n_in, uint32_t n_tok,
-                             uint32_t cus, uint32_t kind);
+uint32_t ah_gemm_pick_splits(uint32_t type, uint32_t n_out, uint32_t n_in, uint32_t n_tok, uint32_t cus,
+                             uint32_t kind, double *cost_us = nullptr);
 uint32_t ah_gemm_part_wg4(uint32_t type, uint32_t n_out, uint32_t n_in, uint32_t n_tok, uint32_t splits,
                           uint32_t kind);
 uint32_t ah_gemm_max_parts(uint32_t type);
@@ -58,6 +58,8 @@ hipError_t ah_launch_gemm_operand(const OperandArgs &o, hipStream_t stream);
 hipError_t ah_launch_swiglu_quant(const SwigluArgs &a, hipStream_t stream);
 size_t ah_few_lds_bytes(uint32_t type, uint32_t kpad, uint32_t tok, uint32_t waves);
 uint32_t ah_few_splits(uint32_t type, uint32_t n_in);
+double ah_few_cost(uint32_t type, uint32_t n_in, uint32_t kpad, uint32_t tok, uint32_t splits, uint32_t waves, size_t wgs,
+                   uint32_t cus);
 hipError_t ah_few_init_attrs();
 hipError_t ah_launch_few(uint32_t type, FewArgs &a, bool ffn, hipStream_t stream);
 hipError_t ah_probe_mfma(uint32_t kind, uint32_t cus, const uint32_t *d_seed, uint32_t *d_sink,
@@ -514,13 +516,28 @@ uint32_t few_tile_of_run(const ah_ctx *ctx, uint32_t tile, size_t wgs) {
 }
 uint32_t few_tok_tile(const ah_ctx *ctx, const ah_tensor *t, size_t n_tok) {
     if (n_tok > kFewTokens || ctx->design[t->type] != AH_GEMM_DESIGN_AUTO) return 0;
-    if (n_tok > 16 && (t->type == AH_GGML_Q4_K || t->type == AH_GGML_Q2_K) &&
-        2 * few_wgs(t->type, t->n_out, t->n_in) > (size_t)ctx->cu_count)
-        return 0;
-    uint32_t tok = n_tok > 16 ? 32u : 16u;
-    while (tok >= 8 && ah_few_lds_bytes(t->type, kpad_of(t->n_in), n_tok < tok ? (uint32_t)n_tok : tok, kFewMaxWaves) > 160 * 1024)
-        tok /= 2;
-    return tok >= 8 && n_tok <= 2 * tok ? tok : 0;
+    const uint32_t n = (uint32_t)n_tok, n_in = (uint32_t)t->n_in, kpad = kpad_of(t->n_in), cus = (uint32_t)ctx->cu_count;
+    const size_t wgs = few_wgs(t->type, t->n_out, t->n_in);
+    if (n > 16 && (t->type == AH_GGML_Q4_K || t->type == AH_GGML_Q2_K) && 2 * wgs > cus) return 0;
+    uint32_t tok = n > 16 ? 32u : 16u;
+    while (tok >= 8 && ah_few_lds_bytes(t->type, kpad, n < tok ? n : tok, kFewMaxWaves) > 160 * 1024) tok /= 2;
+    if (tok < 8 || n > 2 * tok) return 0;
+    // Past one round over the CUs the tile GEMM, whose workgroups read 128 rows for all the tokens, is
+    // the faster one from some size on.  Both costs are models in us (the tile GEMM's is its split
+    // plan's), fitted to the difference of the two at 451 sizes up to 18000 rows where it is small.
+    // us on this route and on the tile GEMM, means of f32 and codes: Q4_K 8960 x 8960 at 12 tokens 57.8 and
+    // 33.5, 4864 x 6144 25.5 and 22.1, at 8 tokens 17.0 and 21.8; Q2_K 8960 x 4864 at 12 40.0 and 32.0; Q8_0
+    // 8960 x 8960 at 12 73.3 and 55.1; Q3_K 8960 x 4864 at 24 59.7 and 38.0, at 8 25.3 and 37.0.  Of 2768 calls
+    // of 5 to 32 tokens at drawn sizes of 1500 to 9000, 115 took over 5% longer than on the tile GEMM (up
+    // to 61%) and 17 do with this line (up to 27%); 14 that took over 5% less now run there.
+    const uint32_t run = few_tile_of_run(ctx, tok, wgs), splits = ah_few_splits(t->type, n_in);
+    const double cost = ah_few_cost(t->type, n_in, kpad, n < run ? n : run, splits, few_waves(splits), wgs * ((n + run - 1) / run), cus);
+    if (cost > 0.0) {
+        double tile = 0.0;
+        ah_gemm_pick_splits(t->type, (uint32_t)t->n_out, n_in, n, cus, ah_k23((int)t->type) ? kGemmKindTile : kGemmKindRb, &tile);
+        if (cost > 8.6 + 0.78 * tile) return 0;
+    }
+    return tok;
 }
 FewArgs few_args(uint32_t src, const void *x, const int64_t *scales, uint32_t n_in, uint32_t n_tok, uint32_t tok_tile,
                  unsigned long long *status) {
@@ -663,17 +680,21 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
     size_t n23 = 0, n_few = 0;
     // Few-token parts: one launch per run of parts of one type.  (The fused FFN form
     // and a part without rows stay below.)
-    auto few = [&](const ah_tensor *t) { return !ffn && t->n_out ? few_tok_tile(ctx, t, n_tok) : 0u; };
-    auto direct = [&](const ah_tensor *t) { return few(t) != 0 || gemv23(t); };
+    uint32_t few_stack[kStackParts];
+    std::vector<uint32_t> few_heap;
+    if (n_parts > kStackParts) few_heap.resize(n_parts);
+    uint32_t *const few = n_parts > kStackParts ? few_heap.data() : few_stack;  // token tile per part (0: not this route)
+    auto direct = [&](size_t i) { return few[i] != 0 || gemv23(w[i]); };
     for (size_t i = 0; i < n_parts; ++i) {
-        n_few += few(w[i]) ? 1 : 0;
-        n23 += !few(w[i]) && gemv23(w[i]) ? 1 : 0;
+        few[i] = !ffn && w[i]->n_out ? few_tok_tile(ctx, w[i], n_tok) : 0u;
+        n_few += few[i] ? 1 : 0;
+        n23 += gemv23(w[i]) ? 1 : 0;
     }
     if (n_few) {
         AH_HIP(ctx, hipSetDevice(ctx->device));
         FewArgs q = {};  // the input once quantized
         for (size_t i = 0; i < n_parts;) {
-            const uint32_t tile = few(w[i]);
+            const uint32_t tile = few[i];
             if (!tile) {
                 ++i;
                 continue;
@@ -685,7 +706,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
             size_t wgs = 0;
             for (; i < n_parts && fa.n_parts < kFewMaxParts; ++i) {
                 if (w[i]->n_out == 0) continue;
-                if (w[i]->type != type || few(w[i]) != tile) break;
+                if (w[i]->type != type || few[i] != tile) break;
                 fa.p[fa.n_parts++] = few_part(w[i], y[i], key0[i]);
                 wgs += few_wgs(type, w[i]->n_out, fa.n_in);
             }
@@ -727,7 +748,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
         const uint32_t kp = kpad_of(n_in_sz);
         AH_HIP(ctx, hipSetDevice(ctx->device));
         for (size_t i = 0; i < n_parts; ++i) {
-            if (few(w[i]) || !gemv23(w[i]) || w[i]->n_out == 0) continue;
+            if (!gemv23(w[i]) || w[i]->n_out == 0) continue;
             // rows that fit the streaming kernel's tile: four tokens per launch, as the argument
             // parts of one launch (each workgroup quantizes its own token's activation), so each
             // launch fills more of the device and the weight rows are re-read from L2
@@ -761,7 +782,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
     }
     if (n_few || n23) {
         size_t n_rest = 0;
-        for (size_t i = 0; i < n_parts; ++i) n_rest += !direct(w[i]) && w[i]->n_out ? 1 : 0;
+        for (size_t i = 0; i < n_parts; ++i) n_rest += !direct(i) && w[i]->n_out ? 1 : 0;
         if (n_few ? n_rest == 0 : n23 == n_parts) return AH_OK;
         const ah_tensor *rw_stack[kStackParts];
         float *ry_stack[kStackParts];
@@ -776,7 +797,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
         float **ry = n_parts > kStackParts ? ry_heap.data() : ry_stack;
         size_t k = 0;
         for (size_t i = 0; i < n_parts; ++i)
-            if (!direct(w[i])) {
+            if (!direct(i)) {
                 rw[k] = w[i];
                 ry[k++] = y[i];
             }
@@ -788,7 +809,7 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
         uint64_t *t0 = n_parts > kStackParts ? t_heap.data() : t_stack;
         size_t q = 0;
         for (size_t i = 0; i < n_parts; ++i)
-            if (!direct(w[i])) t0[q++] = key0[i];
+            if (!direct(i)) t0[q++] = key0[i];
         o2.key0 = t0;
         return gemm_group_launch(ctx, k, rw, src, x, scales_in, n_tok, ry, stream, fixed, fixed_cap, &o2);
     }

@@ -550,6 +550,22 @@ uint32_t ah_few_splits(uint32_t type, uint32_t n_in) {
     return per ? (nu + per - 1) / per : 1;  // the same longest wave with the fewest of them
 }
 
+// us of `wgs` workgroups of `tok` tokens past a launch's fixed time, where they take more than one
+// round over the CUs (0: one round, in which the route was the faster one at every size measured):
+// 5.1 a round, and for each workgroup a CU runs the staging of its tokens and the folds of its
+// units.  A CU holds the workgroups that fit its LDS and the waves that fit its registers: 24 at 80
+// VGPRs, 20 at 87 (Q2_K and Q6_K), 16 with two operand tiles.  ah_abi.cpp compares it with the tile
+// GEMM's.
+double ah_few_cost(uint32_t type, uint32_t n_in, uint32_t kpad, uint32_t tok, uint32_t splits, uint32_t waves, size_t wgs, uint32_t cus) {
+    const size_t by_lds = 160 * 1024 / ah_few_lds_bytes(type, kpad, tok, waves), by_waves = (tok > 16 ? 16 : type == AH_GGML_Q2_K || type == AH_GGML_Q6_K ? 20 : 24) / waves;
+    const size_t held = by_lds < by_waves ? by_lds : by_waves, per_round = cus * (held ? held : 1);
+    const size_t rounds = (wgs + per_round - 1) / per_round;
+    if (rounds <= 1) return 0.0;
+    const uint32_t nu = (n_in + unit_k_of(type) - 1) / unit_k_of(type), per = (nu + splits - 1) / splits;
+    const double fold = type == AH_GGML_Q4_K ? 1.5 : type == AH_GGML_Q2_K ? 1.13 : type == AH_GGML_Q6_K ? 0.75 : type == AH_GGML_Q3_K ? 0.32 : 0.46;
+    return 5.1 * (double)rounds + (double)((wgs + cus - 1) / cus) * (0.24e-4 * tok * kpad + fold * (waves * per * (tok > 16 ? 2 : 1)) / 16.0);
+}
+
 hipError_t ah_few_init_attrs() {
     for (uint32_t t : {AH_GGML_Q8_0, AH_GGML_Q5_0, AH_GGML_Q2_K, AH_GGML_Q3_K, AH_GGML_Q4_K, AH_GGML_Q6_K})
         for (uint32_t nt = 1; nt <= 2; ++nt)

@@ -1943,7 +1943,7 @@ uint32_t per_split(const GemmGeom &g, uint32_t splits) {
 //   a split GEMM adds the reduction: 4.8 us fixed plus the partials' write and read-back,
 //   (splits + 1) * n_tok * n_out * 4 bytes at 0.253 us per MB.
 uint32_t ah_gemm_pick_splits(uint32_t type, uint32_t n_out, uint32_t n_in, uint32_t n_tok,
-                             uint32_t cus, uint32_t kind) {
+                             uint32_t cus, uint32_t kind, double *cost_us) {
     const bool int8 = kind == kGemmKindI8;
     const GemmGeom g = geom_of(type, n_in, (n_in + 255) / 256 * 256, 4, kind);
     const uint64_t tiles = (uint64_t)((n_out + g.rows - 1) / g.rows) * ((n_tok + g.toks - 1) / g.toks);
@@ -1962,6 +1962,7 @@ uint32_t ah_gemm_pick_splits(uint32_t type, uint32_t n_out, uint32_t n_in, uint3
             best = used;
         }
     }
+    if (cost_us) *cost_us = best_cost;
     return best;
 }
 

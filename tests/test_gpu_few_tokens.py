@@ -186,3 +186,31 @@ def test_few_tokens_code_rows_at_any_byte(dev, t, n_in):
             assert dev.sync_status(stream()) == 0
             assert torch.equal(yq, y), (n_tok, off)
     w.free()
+
+
+@pytest.mark.parametrize("t,n_out,n_in,n_tok,route", [
+    (Q4_K, 1536, 8960, 12, "few"), (Q4_K, 2560, 8960, 12, "tile"), (Q4_K, 4864, 6144, 12, "tile"), (Q4_K, 4864, 6144, 4, "few"),
+    (Q2_K, 4200, 8960, 12, "tile"), (Q3_K, 4200, 4864, 24, "tile"), (Q3_K, 4200, 4864, 12, "few"), (Q8_0, 4400, 8960, 12, "tile"),
+    (Q8_0, 4400, 8960, 8, "few"), (Q6_K, 9000, 4864, 24, "tile"), (Q6_K, 9000, 4864, 12, "few"), (Q5_0, 9000, 4864, 32, "tile"),
+])
+def test_wide_calls_keep_the_tile_gemm(dev, t, n_out, n_in, n_tok, route):
+    """Where the few-token kernel's rounds over the CUs take longer than the tile GEMM, AUTO is the tile
+    GEMM, from f32 and from codes: the outputs of the design that names it, bit for bit."""
+    rng = synth.rng_for(14, n_out + n_in + t)
+    w = dev.upload(t, payload(t, rng, n_out, n_in), n_out, n_in)
+    dx = torch.from_numpy(synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)).cuda()
+    dc = torch.zeros((n_tok, n_in), dtype=torch.int8, device="cuda")
+    ds = torch.zeros((n_tok, n_in // 32), dtype=torch.int64, device="cuda")
+    dev.quant_act_f32_dev(dx.data_ptr(), n_tok, n_in, dc.data_ptr(), ds.data_ptr(), stream())
+    y, yq, named = (torch.full((n_tok, n_out), float("nan"), device="cuda") for _ in range(3))
+    w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+    w.gemm_q8_dev(dc.data_ptr(), ds.data_ptr(), n_tok, yq.data_ptr(), stream())
+    dev.set_gemm_design(t, 3 if t in (Q2_K, Q3_K) else 1)
+    try:
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, named.data_ptr(), stream())
+        assert dev.sync_status(stream()) == 0
+    finally:
+        dev.set_gemm_design(t, 0)
+    assert torch.equal(y, yq)
+    assert torch.equal(y, named) == (route == "tile")
+    w.free()

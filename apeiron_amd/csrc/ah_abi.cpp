@@ -539,6 +539,17 @@ uint32_t few_tok_tile(const ah_ctx *ctx, const ah_tensor *t, size_t n_tok) {
     }
     return tok;
 }
+// The few-token kernel's workgroups read the call's input while others write its outputs, so a call
+// whose outputs lie over its input (y over x) keeps the tile GEMM, whose operand pass has read all of
+// the input before the first output is written.
+bool few_over(const void *out, size_t bytes, uint32_t src, const void *x, const void *scales, size_t n_tok, size_t n_in) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out);
+    auto over = [&](const void *p, size_t len) {
+        const uintptr_t i = reinterpret_cast<uintptr_t>(p);
+        return out && p && o < i + len && i < o + bytes;
+    };
+    return over(x, n_tok * n_in * (src == AH_SRC_F32 ? 4 : 1)) || (src == AH_SRC_CODES && over(scales, n_tok * ((n_in + 31) / 32) * 8));
+}
 FewArgs few_args(uint32_t src, const void *x, const int64_t *scales, uint32_t n_in, uint32_t n_tok, uint32_t tok_tile,
                  unsigned long long *status) {
     FewArgs a;
@@ -685,8 +696,11 @@ int32_t gemm_group_launch(ah_ctx *ctx, size_t n_parts, const ah_tensor *const *w
     if (n_parts > kStackParts) few_heap.resize(n_parts);
     uint32_t *const few = n_parts > kStackParts ? few_heap.data() : few_stack;  // token tile per part (0: not this route)
     auto direct = [&](size_t i) { return few[i] != 0 || gemv23(w[i]); };
+    bool over = false;
+    for (size_t i = 0; i < n_parts && n_tok <= kFewTokens; ++i)
+        over = over || few_over(y[i], n_tok * w[i]->n_out * 4, src, x, scales_in, n_tok, n_in_sz);
     for (size_t i = 0; i < n_parts; ++i) {
-        few[i] = !ffn && w[i]->n_out ? few_tok_tile(ctx, w[i], n_tok) : 0u;
+        few[i] = !ffn && !over && w[i]->n_out ? few_tok_tile(ctx, w[i], n_tok) : 0u;
         n_few += few[i] ? 1 : 0;
         n23 += gemv23(w[i]) ? 1 : 0;
     }
@@ -1359,9 +1373,13 @@ static int32_t ffn_prefill_gate_up(ah_ctx *ctx, const ah_tensor *gate, const ah_
     }
     if (n_ff > (0xFFFFFF00ull / (128 * 4))) return AH_ERR_INVALID_ARG;  // as gemm_group_launch refuses it
     // a few tokens: one launch, the SwiGLU in its epilogue (a workgroup is the K splits of two row
-    // tiles of each projection, so at most four splits)
+    // tiles of each projection, so at most four splits); no output over the input, as in a group
     const uint32_t ffn_splits = ah_few_splits(t, (uint32_t)gate->n_in);
-    if (const uint32_t tile = ctx->ffn_form == AH_FFN_PREFILL_AUTO && 4 * ffn_splits <= kFewMaxWaves ? few_tok_tile(ctx, gate, n_tok) : 0) {
+    auto over = [&](const void *out, size_t bytes) { return few_over(out, bytes, src, d_x, d_scales, n_tok, gate->n_in); };
+    const bool few = ctx->ffn_form == AH_FFN_PREFILL_AUTO && 4 * ffn_splits <= kFewMaxWaves && n_tok <= kFewTokens &&
+                     !over(d_gate_y, n_tok * n_ff * 4) && !over(d_up_y, n_tok * n_ff * 4) && !over(d_h_codes, n_tok * n_ff) &&
+                     !over(d_h_scales, n_tok * ((n_ff + 31) / 32) * 8);
+    if (const uint32_t tile = few ? few_tok_tile(ctx, gate, n_tok) : 0) {
         FewArgs fa = few_args(src, d_x, d_scales, (uint32_t)gate->n_in, (uint32_t)n_tok, tile, ctx->d_status);
         fa.n_parts = 2;
         fa.p[0] = few_part(gate, nullptr, 0);

@@ -214,3 +214,51 @@ def test_wide_calls_keep_the_tile_gemm(dev, t, n_out, n_in, n_tok, route):
     assert torch.equal(y, yq)
     assert torch.equal(y, named) == (route == "tile")
     w.free()
+
+
+@pytest.mark.parametrize("t", ALL)
+def test_outputs_over_the_input(dev, t):
+    """An output that lies over the call's input: the input is read whole before anything is written, so
+    the call gives what it gives with separate buffers on the tile GEMM."""
+    n, n_tok, n_ff = 512, 9, 512
+    rng = synth.rng_for(15, t)
+    W = [dev.upload(t, payload(t, rng, n, n), n, n) for _ in range(3)]
+    x = torch.from_numpy(synth.activations(rng, n, n_tok).reshape(n_tok, n)).cuda() * 2.0 ** -4
+    codes, scales = torch.zeros((n_tok, n), dtype=torch.int8, device="cuda"), torch.zeros((n_tok, n // 32), dtype=torch.int64, device="cuda")
+    dev.quant_act_f32_dev(x.data_ptr(), n_tok, n, codes.data_ptr(), scales.data_ptr(), stream())
+    new = lambda: torch.full((n_tok, n), float("nan"), device="cuda")  # noqa: E731
+    # one projection, then three of which the second's output is the input
+    ref = [new() for _ in W]
+    dev.set_gemm_design(t, 3 if t in (Q2_K, Q3_K) else 1)
+    try:
+        for w, y in zip(W, ref):
+            w.gemm_f32_dev(x.data_ptr(), n_tok, y.data_ptr(), stream())
+        assert dev.sync_status(stream()) == 0
+    finally:
+        dev.set_gemm_design(t, 0)
+    y = x.clone()
+    W[0].gemm_f32_dev(y.data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0 and torch.equal(y, ref[0])
+    y0, y1, y2 = new(), x.clone(), new()
+    chart.gemm_group_f32_dev(dev, W, y1.data_ptr(), n_tok, [q.data_ptr() for q in (y0, y1, y2)], stream())
+    assert dev.sync_status(stream()) == 0
+    assert all(torch.equal(q, r) for q, r in zip((y0, y1, y2), ref))
+    # from codes inside the output's buffer
+    y = new()
+    held = y.view(torch.int8).reshape(-1)[:n_tok * n]
+    held.copy_(codes.reshape(-1))
+    W[0].gemm_q8_dev(held.data_ptr(), scales.data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0 and torch.equal(y, ref[0])
+    # the FFN's hidden codes over its input, f32 and codes
+    hc, hs = torch.zeros((n_tok, n_ff), dtype=torch.int8, device="cuda"), torch.zeros((n_tok, n_ff // 32), dtype=torch.int64, device="cuda")
+    chart.ffn_gate_up_prefill_dev(dev, W[0], W[1], x.data_ptr(), n_tok, hc.data_ptr(), hs.data_ptr(), stream=stream())
+    out, held, hs2 = new(), x.clone(), torch.zeros_like(hs)
+    chart.ffn_gate_up_prefill_dev(dev, W[0], W[1], held.data_ptr(), n_tok, held.data_ptr(), hs2.data_ptr(), stream=stream())
+    assert dev.sync_status(stream()) == 0
+    assert torch.equal(held.view(torch.int8).reshape(-1)[:n_tok * n_ff], hc.reshape(-1)) and torch.equal(hs2, hs)
+    c2, s2 = codes.clone(), scales.clone()
+    chart.ffn_prefill_q8_dev(dev, W[0], W[1], W[2], c2.data_ptr(), s2.data_ptr(), n_tok, out.data_ptr(), c2.data_ptr(), s2.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0
+    assert torch.equal(c2, hc) and torch.equal(s2, hs)
+    for w in W:
+        w.free()

@@ -1,9 +1,10 @@
 """GPU parity of the few-token GEMM (calls of at most 32 tokens) through the C ABI, at the sizes where
 it can go wrong: every family, one to 32 tokens around its 16-token operand tiles, widths off its
 16-row tiles, K around its units of 128 / 256 and its waves' K splits, rows too long for one tile's
-LDS (two token tiles, then the tile GEMM), f32 inputs quantized in the kernel and by a launch of
-their own, code rows off dword boundaries, payloads that end at their last byte, the SwiGLU epilogue
-of the prefill FFN, and a QuantAct scale whose products leave int64.
+LDS (two token tiles, then the tile GEMM), sizes whose rounds over the CUs leave it for the tile
+GEMM, f32 inputs quantized in the kernel and by a launch of their own, code rows off dword boundaries,
+groups of parts, outputs over the input, payloads that end at their last byte, the SwiGLU epilogue of
+the prefill FFN, and a QuantAct scale whose products leave int64.
 
 Tolerance: every 32-block (or super-block half) is one exact integer dot folded with at most four
 f32 roundings, and the blocks' sums with one each, so an output is within (blocks + 8) * 2^-24 of the
@@ -56,7 +57,7 @@ def close(t, raw, n_out, n_in, codes, scales, y, what):
 @pytest.mark.parametrize("n_tok,n_out,n_in", [
     (1, 16, 32), (2, 17, 256), (8, 130, 300), (9, 48, 901), (16, 33, 1536), (17, 40, 1000), (32, 129, 520),
     (3, 20, 4864), (16, 18, 8960),   # waves of several units; two tiles of 8 tokens
-    (2, 16, 32768),                  # past the LDS: the tile GEMM
+    (2, 16, 32768),                  # the longest rows
 ])
 def test_few_tokens_vs_oracle(dev, t, n_tok, n_out, n_in):
     rng = synth.rng_for(9, 1000 * t + n_in + n_tok)
@@ -81,6 +82,75 @@ def test_few_tokens_vs_oracle(dev, t, n_tok, n_out, n_in):
             w.gemm_q8_dev(dc.data_ptr() + off, ds.data_ptr(), n_tok, yq.data_ptr(), stream())
             assert dev.sync_status(stream()) == 0
             assert (yq == y).all(), (off, int((yq != y).sum()))
+        w.free()
+
+
+# The longest rows whose 16 (two tiles of 8) and 32 (two of 16) tokens fit a CU's LDS.
+LDS_ROWS = {Q5_0: (14848, 7424), Q8_0: (13056, 6400), Q2_K: (12032, 5888), Q3_K: (14080, 6912), Q4_K: (12544, 6144), Q6_K: (11264, 5632)}
+
+
+@pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("n_tok", [16, 32])
+def test_rows_at_the_lds_limit(dev, t, n_tok):
+    """At the longest rows that fit the call runs on the few-token kernel, 256 columns further on the
+    tile GEMM (the bits of the design that names it); both hold the oracle's bound."""
+    n_out = 20
+    for n_in, few in ((LDS_ROWS[t][n_tok > 16], True), (LDS_ROWS[t][n_tok > 16] + 256, False)):
+        rng = synth.rng_for(16, n_in + t)
+        raw = payload(t, rng, n_out, n_in)
+        w = dev.upload(t, raw, n_out, n_in)
+        x = synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)
+        dx = torch.from_numpy(x).cuda()
+        y, named = (torch.full((n_tok, n_out), float("nan"), device="cuda") for _ in range(2))
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+        dev.set_gemm_design(t, 3 if t in (Q2_K, Q3_K) else 1)
+        try:
+            w.gemm_f32_dev(dx.data_ptr(), n_tok, named.data_ptr(), stream())
+            assert dev.sync_status(stream()) == 0
+        finally:
+            dev.set_gemm_design(t, 0)
+        assert torch.equal(y, named) != few, n_in
+        st, codes, scales = oracle.quant_act_f32_batch(x)
+        assert st == 0
+        if few:
+            close(t, raw, n_out, n_in, codes, scales, y.cpu().numpy(), f"K {n_in}")
+        w.free()
+
+
+GROUPS = {  # (type, n_out) of the parts
+    "qkv": [(Q4_K, 1536), (Q4_K, 256), (Q6_K, 256)],
+    "wide": [(Q4_K, 8960), (Q6_K, 300), (Q8_0, 0), (Q8_0, 64)],  # at 24 tokens its Q4_K part keeps the tile GEMM
+    "six": [(Q8_0, 96), (Q8_0, 17), (Q8_0, 0), (Q8_0, 130), (Q8_0, 64), (Q8_0, 33), (Q8_0, 300)],  # two launches
+    "types": [(Q3_K, 130), (Q5_0, 64), (Q2_K, 33), (Q3_K, 64), (Q6_K, 40)],
+}
+
+
+@pytest.mark.parametrize("group", sorted(GROUPS))
+@pytest.mark.parametrize("n_tok", [9, 16, 24])
+@pytest.mark.parametrize("src", ["f32", "codes"])
+def test_grouped_parts_are_their_single_calls(dev, group, n_tok, src):
+    """Parts of several types, an input quantized once for all of them, more parts of a type than a launch
+    holds, parts without rows and parts of both routes: each is its single call's output bit for bit."""
+    n_in = 1536
+    rng = synth.rng_for(17, n_tok + len(group))
+    ws = [dev.upload(t, payload(t, rng, o, n_in), o, n_in) for t, o in GROUPS[group]]
+    dx = torch.from_numpy(synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)).cuda()
+    dc = torch.zeros((n_tok, n_in), dtype=torch.int8, device="cuda")
+    ds = torch.zeros((n_tok, n_in // 32), dtype=torch.int64, device="cuda")
+    dev.quant_act_f32_dev(dx.data_ptr(), n_tok, n_in, dc.data_ptr(), ds.data_ptr(), stream())
+    ys, y1 = ([torch.full((n_tok, max(w.n_out, 1)), float("nan"), device="cuda") for w in ws] for _ in range(2))
+    if src == "f32":
+        chart.gemm_group_f32_dev(dev, ws, dx.data_ptr(), n_tok, [y.data_ptr() for y in ys], stream())
+    else:
+        chart.gemm_group_q8_dev(dev, ws, dc.data_ptr(), ds.data_ptr(), n_tok, [y.data_ptr() for y in ys], stream())
+    for w, y in zip(ws, y1):
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0
+    for w, y, one in zip(ws, ys, y1):
+        if w.n_out:
+            assert torch.isfinite(y).all() and torch.equal(y, one), (w.n_out, group)
+        else:
+            assert torch.isnan(y).all()
         w.free()
 
 

@@ -188,9 +188,9 @@ def const_payload(t, n_out, n_in, d_bits):
     return blk.reshape(-1)
 
 
-@pytest.mark.parametrize("t,fused", [(Q4_K, True), (Q4_K, False), (Q8_0, True)])
+@pytest.mark.parametrize("t,fused", [(Q4_K, True), (Q4_K, False), (Q8_0, True), (Q4_K, None), (Q8_0, None)])
 def test_ffn_prefill_refusal_order(dev, t, fused):
-    """Refusals in the order the reference meets them, not token-major: every token's gate output
+    """(fused None: AUTO, here the few-token kernel with the SwiGLU in its epilogue.)  Refusals in the order the reference meets them, not token-major: every token's gate output
     before any up output, those before any SwiGLU element, and the down projection last; the
     input's quantization before all of them."""
     n_embd, n_ff = 256, 64
@@ -208,7 +208,8 @@ def test_ffn_prefill_refusal_order(dev, t, fused):
         chart.ffn_gate_up_prefill_dev(dev, G, U, x.data_ptr(), 2, hc.data_ptr(), hs.data_ptr(), None, None, stream())
         return dev.sync_status(stream())
 
-    dev.set_ffn_prefill_form(chart.Device.FFN_FUSED if fused else chart.Device.FFN_TWO_PASS)
+    dev.set_ffn_prefill_form(chart.Device.FFN_AUTO if fused is None else
+                             chart.Device.FFN_FUSED if fused else chart.Device.FFN_TWO_PASS)
     try:
         # token 0: gate = up = 2^16, h = 2^32 leaves i64 (SwiGLU refusal, 12); token 1: gate = up =
         # 2^32 (OutputOverflow, 9).  The gate projection of token 1 comes first.

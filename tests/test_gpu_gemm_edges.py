@@ -13,8 +13,8 @@ reference's LCG stream is not needed: the distributions are what the tests exerc
   left by 29*b/(groups-1), for Q4_K / Q6_K / Q8_0 at n_out = 7, n_in in {256, 1024}.
 * tests/golden/golden.npz: every fixture through the GEMM.
 * A token whose largest blocks meet zero weights while the row's weight sits on blocks 2^27
-  lower: under a per-token f16 band those blocks would be lost (the whole result), so the operand
-  pass must route the token to the exact path.
+  lower: under a per-token f16 band those blocks would be lost (the whole result), so the tile
+  GEMM's operand pass must route the token to the exact path.
 * chart/tests.rs:525-560 ``chart_agrees_with_fixed_on_every_refusal_class``: each refusal class
   through the GPU forms.
 
@@ -46,6 +46,19 @@ def dev():
     d = chart.Device(0)
     yield d
     d.close()
+
+
+@pytest.fixture(params=["auto", "tile"])
+def route(dev, request):
+    """Calls of at most 32 tokens on the route AUTO picks (mostly the few-token kernel, which has no f16
+    band and no exact path) and on the tile GEMM that longer calls take."""
+    designs = {6: 1, 8: 1, 10: 3, 11: 3, 12: 1, 14: 1}
+    if request.param == "tile":
+        for t, design in designs.items():
+            dev.set_gemm_design(t, design)
+    yield request.param
+    for t in designs:
+        dev.set_gemm_design(t, 0)
 
 
 def stream():
@@ -175,6 +188,7 @@ def check_call(t, raw, n_out, n_in, codes, scales, st_gpu, Y, what):
 
 # ---- tests -----------------------------------------------------------------------------------
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("n_out,n_in", [(1, 32), (17, 64), (33, 1024), (40, 3584)])
 def test_gemm_reference_equality_inputs(dev, n_out, n_in):
     """kern/gemm.rs:2607-2645 on the GPU GEMM (codes input), with GEMM(N=1) = GEMV on each."""
@@ -198,6 +212,7 @@ def test_gemm_reference_equality_inputs(dev, n_out, n_in):
         assert refusals > 0  # the largest scale word drives some calls past 2^31
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("t", [12, 14, 8, 6])
 @pytest.mark.parametrize("n_in", [256, 1024])
 def test_gemm_spread_columns(dev, t, n_in):
@@ -212,6 +227,7 @@ def test_gemm_spread_columns(dev, t, n_in):
     w.free()
 
 
+@pytest.mark.usefixtures("route")
 def test_gemm_golden_fixtures(dev):
     """Every golden fixture as a GEMM: its column, a zero column and its column again."""
     z = np.load(GOLDEN, allow_pickle=False)
@@ -263,11 +279,12 @@ def cliff_case(t, n_in, gap, rng):
     return R.reshape(-1), x
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("t", [6, 8, 12, 14])
 @pytest.mark.parametrize("gap", [27, 24, 20, 12])
 def test_gemm_zero_weight_heavy_blocks(dev, t, gap):
-    """Heavy blocks against zero weights, the rest 2^gap lower.  gap 27 is past the f16 band
-    (the token takes the exact path); gap 24 and 20 keep it on the MFMA with subnormal f16
+    """Heavy blocks against zero weights, the rest 2^gap lower.  On the tile GEMM, gap 27 is past the f16
+    band (the token takes the exact path) and gap 24 and 20 keep it on the MFMA with subnormal f16
     operands (exact at 2^-24 and above); the GEMM equals the oracle and the GEMV either way."""
     rng = np.random.default_rng(1000 * t + gap)
     n_in = 1024
@@ -285,10 +302,11 @@ def test_gemm_zero_weight_heavy_blocks(dev, t, gap):
     w.free()
 
 
+@pytest.mark.usefixtures("route")
 @pytest.mark.parametrize("t", [6, 8, 12, 14])
 def test_gemm_f32_input_wide_spread_tokens(dev, t):
-    """f32 input whose blocks span ~40 binades (flagged by the operand pass, whose quantized codes
-    it keeps for the exact path) mixed with ordinary tokens, at a split-K shape and a small one."""
+    """f32 input whose blocks span ~40 binades (flagged by the tile GEMM's operand pass, whose quantized
+    codes it keeps for the exact path) mixed with ordinary tokens, at a split-K shape and a small one."""
     rng = np.random.default_rng(77 + t)
     for n_out, n_in, n_tok in ((1536, 8960, 70), (96, 512, 9)):
         raw = synth.payload(t, rng, n_out, n_in)
@@ -349,6 +367,7 @@ def test_gemm_exact_path_every_row_to_the_payload_end(dev, t):
         w.free()
 
 
+@pytest.mark.usefixtures("route")
 def test_refusal_classes_match_reference(dev):
     """chart/tests.rs:525-560 through the GPU forms: each refusal class gives the contract's."""
     rng = np.random.default_rng(7)
@@ -412,9 +431,10 @@ def test_refusal_classes_match_reference(dev):
     w_1.free()
 
 
+@pytest.mark.usefixtures("route")
 def test_gemm_odd_scale_quantacts(dev):
     """Hand-built QuantActs whose scales are not powers of two (any i64 the reference accepts that
-    dequantizes): the GEMM serves them on the exact path and matches the GEMV and the contract."""
+    dequantizes): the tile GEMM serves them on the exact path; both routes match the contract."""
     rng = np.random.default_rng(11)
     for t in (8, 12, 14):
         n_out, n_in = 40, 512
@@ -443,12 +463,13 @@ def big_k23_payload(t, n_out, n_in):
 
 
 @pytest.mark.parametrize("t", [10, 11])
-@pytest.mark.parametrize("design", [0, 1])
+@pytest.mark.parametrize("design", [0, 1, 3])
 def test_k23_refusal_order_across_tokens(dev, t, design):
     """The first refusal of a prefill is the first refusing column's (chart/mod.rs:1955-1975 runs
     matvec_q8act column by column), also when a later column refuses at an earlier row with a
     smaller code: OutputOverflow (9) of column 0 wins over AccumulatorOverflow (8) of column 1
-    and the reverse.  Q2_K / Q3_K through the tiles (AUTO) and the per-token GEMV route (F16)."""
+    and the reverse.  Q2_K / Q3_K through AUTO (here the few-token kernel), the per-token GEMV route
+    (F16) and the tiles (F16_TILE)."""
     n_out, n_in = 3, 4096
     raw = big_k23_payload(t, n_out, n_in)
     w = dev.upload(t, raw, n_out, n_in)
@@ -525,6 +546,38 @@ def test_token_tile_chunks(dev, t, n_out, n_in, n_tok, form):
         err = np.abs(same[0].astype(np.float64) - ref.astype(np.float64) * Q32)
         assert (err <= TOL * absdot + Q32).all(), (c, err.max())
     w.free()
+
+
+def test_token_tile_chunks_in_the_mixed_kernel(dev):
+    """Q4_K and Q6_K parts of one input in one grid, the Q6_K part's 12 token tiles in three chunks: its
+    bits are the single call's, and equal tokens have equal outputs."""
+    rng = synth.rng_for(11, 77)
+    n_in, n_tok, shapes = 8960, 1409, [(12, 100), (14, 512)]
+    base = synth.activations(rng, n_in, 64).reshape(64, n_in)
+    i = np.arange(n_tok)
+    order = (37 * i + i // 64) % 64
+    dx = to_dev(base[order])
+    raws = [synth.q4_k_centered_payload(rng, o, n_in) if t == 12 else synth.payload(t, rng, o, n_in) for t, o in shapes]
+    ws = [dev.upload(t, raw, o, n_in) for (t, o), raw in zip(shapes, raws)]
+    ys, y1 = ([torch.full((n_tok, o), float("nan"), dtype=torch.float32, device="cuda") for _, o in shapes] for _ in range(2))
+    chart.gemm_group_f32_dev(dev, ws, dx.data_ptr(), n_tok, [y.data_ptr() for y in ys], stream())
+    for w, y in zip(ws, y1):
+        w.gemm_f32_dev(dx.data_ptr(), n_tok, y.data_ptr(), stream())
+    assert dev.sync_status(stream()) == 0
+    for (t, o), raw, w, y, one in zip(shapes, raws, ws, ys, y1):
+        assert torch.equal(y, one), t
+        Y = y.cpu().numpy()
+        for c in range(64):
+            same = Y[order == c]
+            assert (same.view(np.int32) == same[0].view(np.int32)).all(), (t, c)
+        for c in (0, 63):
+            st, codes, scales = oracle.quant_act_f32(base[c])
+            st1, ref = oracle.matvec_q8act(t, raw, o, n_in, codes, scales)
+            st2, absdot = oracle.row_absdot(t, raw, o, n_in, codes, scales)
+            assert st == 0 and st1 == 0 and st2 == 0
+            err = np.abs(Y[order == c][0].astype(np.float64) - ref.astype(np.float64) * Q32)
+            assert (err <= TOL * absdot + Q32).all(), (t, c, err.max())
+        w.free()
 
 
 @pytest.mark.parametrize("n_in", [33, 901, 1537, 2049, 4866, 8957])

@@ -545,12 +545,14 @@ def test_mfma_probe_within_published_peaks(dev):
 
 
 @pytest.mark.parametrize("t", [6, 8, 10, 11, 12, 14])
-@pytest.mark.parametrize("n_out,n_in,n_tok", [(96, 301, 5), (130, 8960, 70), (64, 20000, 3), (256, 1536, 129)])
+@pytest.mark.parametrize("n_out,n_in,n_tok", [(96, 301, 5), (96, 301, 37), (130, 8960, 70), (64, 20000, 3), (64, 20000, 33),
+                                              (256, 1536, 129)])
 def test_gemm_codes_input_equals_f32_input(dev, t, n_out, n_in, n_tok):
     """The codes-input GEMM (quantizer output handed over) equals the f32-input GEMM bit for bit:
-    both build the same f16 operand from the same codes.  Covers bytewise code rows (n_in % 4 != 0),
-    and the operand pass's 256-thread form and its 1024-thread forms of 2 and 4 register rounds
-    (K = 8960, 20000); a few columns are checked against the oracle."""
+    past 32 tokens both build the same f16 operand from the same codes, up to 32 the few-token kernel
+    quantizes or reads the same codes.  Covers code rows off the dword grid (n_in % 4 != 0), and the
+    operand pass's 256-thread form and its 1024-thread forms of 2 and 4 register rounds (K = 8960,
+    20000); a few columns are checked against the oracle."""
     rng = synth.rng_for(3, 4000 + t + n_in)
     raw = synth.payload(t, rng, n_out, n_in)
     x = synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)

@@ -88,6 +88,31 @@ def test_group_gemm_refusal_in_part_order(dev, t, design):
             w.free()
 
 
+def test_group_of_both_routes_refusal_in_part_order(dev):
+    """24 tokens of a wide Q4_K part, which keeps the tile GEMM, beside a narrow Q3_K part on the few-token
+    kernel, launched first: the earlier part's refusal wins, whichever route it is on."""
+    n_tok, shape = 24, {Q4_K: 2064, Q3_K: 3}
+    codes = np.full((n_tok, N_IN), 1, np.int8)
+    scales = np.full((n_tok, N_IN // 32), 1 << 20, np.int64)
+    codes[20], scales[20] = 127, 1 << 56
+    dc, ds = torch.from_numpy(codes).cuda(), torch.from_numpy(scales).cuda()
+    raws = {(t, b): const_payload(t, shape[t], b) for t in shape for b in (SMALL, BIG)}
+    W = {k: dev.upload(k[0], r, shape[k[0]], N_IN) for k, r in raws.items()}
+    try:
+        for order in (((Q4_K, SMALL), (Q3_K, BIG)), ((Q4_K, BIG), (Q3_K, SMALL)), ((Q3_K, SMALL), (Q4_K, BIG)),
+                      ((Q3_K, BIG), (Q4_K, SMALL))):
+            t, b = order[0]
+            want, _ = oracle.matvec_q8act(t, const_payload(t, 1, b), 1, N_IN, codes[20], scales[20])
+            assert want == (9 if b == SMALL else 8)
+            ys = [torch.empty((n_tok, shape[k[0]]), dtype=torch.float32, device="cuda") for k in order]
+            chart.gemm_group_q8_dev(dev, [W[k] for k in order], dc.data_ptr(), ds.data_ptr(), n_tok, [y.data_ptr() for y in ys],
+                                    stream())
+            assert dev.sync_status(stream()) == want, order
+    finally:
+        for w in W.values():
+            w.free()
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q3_K])
 def test_gemv_plan_refusal_in_part_order(dev, t):
     """A decode plan over two projections of one input: part order, then row."""

@@ -78,16 +78,35 @@ def test_noalloc_gemm_refuses_past_its_scratch(dev):
 
 @pytest.mark.parametrize("t", [10, 11])
 def test_noalloc_gemm_q2_k_q3_k_route(dev, t):
-    """The Q2_K / Q3_K prefill route (GEMV launches of four tokens' argument parts) through the
-    no-alloc entry point equals the ordinary one bit for bit, on two calls in a row, the second
-    with a smaller input."""
+    """The Q2_K / Q3_K prefill routes (AUTO's few-token kernel, GEMV launches of four tokens' argument
+    parts under F16, the tiles) through the no-alloc entry point equal the ordinary one bit for bit, on
+    two calls in a row, the second with a smaller input."""
     L = dev.lib
-    for n_out, n_in, n_tok in ((300, 896, 9), (64, 512, 3)):
-        rng = synth.rng_for(12, t * 10 + n_tok)
+    for design in (0, 1, 3):
+        dev.set_gemm_design(t, design)
+        try:
+            for n_out, n_in, n_tok in ((300, 896, 9), (64, 512, 3)):
+                rng = synth.rng_for(12, t * 10 + n_tok)
+                w = dev.upload(t, synth.payload(t, rng, n_out, n_in), n_out, n_in)
+                x = torch.from_numpy(synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)).cuda()
+                y1 = run(dev, L.ah_gemm_f32_dev, w, x)
+                y2 = run(dev, L.ah_gemm_f32_noalloc_dev, w, x)
+                assert torch.isfinite(y1).all() and torch.equal(y1, y2)
+                w.free()
+        finally:
+            dev.set_gemm_design(t, chart.Device.GEMM_AUTO)
+
+
+@pytest.mark.parametrize("t", [6, 8, 10, 11, 12, 14])
+def test_noalloc_gemm_few_tokens(dev, t):
+    """Calls of at most 32 tokens: long rows, quantized by a launch of their own into the fixed scratch,
+    then rows that the kernel quantizes itself."""
+    for n_out, n_in, n_tok in ((64, 8960, 16), (40, 1536, 24), (40, 256, 5)):
+        rng = synth.rng_for(14, t * 10 + n_tok)
         w = dev.upload(t, synth.payload(t, rng, n_out, n_in), n_out, n_in)
         x = torch.from_numpy(synth.activations(rng, n_in, n_tok).reshape(n_tok, n_in)).cuda()
-        y1 = run(dev, L.ah_gemm_f32_dev, w, x)
-        y2 = run(dev, L.ah_gemm_f32_noalloc_dev, w, x)
+        y1 = run(dev, dev.lib.ah_gemm_f32_dev, w, x)
+        y2 = run(dev, dev.lib.ah_gemm_f32_noalloc_dev, w, x)
         assert torch.isfinite(y1).all() and torch.equal(y1, y2)
         w.free()
 

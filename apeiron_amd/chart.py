@@ -98,7 +98,8 @@ class Device:
 
     def set_gemm_design(self, ggml_type: int, design: int) -> None:
         """The prefill GEMM design of `ggml_type` on this context (ah_set_gemm_design).  AUTO is
-        F16 for every type but Q2_K and Q3_K, where it is F16_TILE (the dequantize-once tiles);
+        F16 for every type but Q2_K and Q3_K, where it is F16_TILE (the dequantize-once tiles), and up
+        to 32 tokens a one-launch kernel of its own where that is the faster one;
         INT8 exists for Q8_0 and Q4_K, F16_TILE for Q4_K, Q2_K and Q3_K; F16 on Q2_K / Q3_K serves the
         prefill as one streaming GEMV per token."""
         _check(self.lib.ah_set_gemm_design(self.h, ggml_type, design), "set_gemm_design")
@@ -106,8 +107,8 @@ class Device:
     FFN_AUTO, FFN_FUSED, FFN_TWO_PASS = 0, 1, 2
 
     def set_ffn_prefill_form(self, form: int) -> None:
-        """The prefill FFN's form (ah_set_ffn_prefill_form): AUTO (two passes), FUSED (one launch
-        for Q4_K / Q2_K / Q3_K gate/up) or TWO_PASS."""
+        """The prefill FFN's form (ah_set_ffn_prefill_form): AUTO (two passes, or one
+        launch of a few tokens), FUSED (one launch for Q4_K / Q2_K / Q3_K gate/up) or TWO_PASS."""
         _check(self.lib.ah_set_ffn_prefill_form(self.h, form), "set_ffn_prefill_form")
 
     def probe_mfma_peak(self, kind: int) -> float:

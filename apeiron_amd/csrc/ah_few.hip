@@ -5,7 +5,8 @@
 // on token c.  At 2 to 32 tokens the weights are still read once per call, as in a GEMV, and what
 // bounds the call is latency: the operand pass, the K loop of a tile made for 64 or 128 tokens and
 // the split-K reduction were three dependent launches of 4 to 23 us each.  Here one launch does all
-// of it.  A workgroup is 16 waves: R row tiles of 16 weight rows, S waves along K for each.
+// of it.  A workgroup is up to 16 waves: S along K (ah_few_splits) for each of R row tiles of 16
+// weight rows, 5 to 8 waves where S is below 8; with the SwiGLU epilogue four row tiles, 4 S waves.
 //   * The workgroup quantizes its tokens' activations into LDS itself (the GEMV's quantizer; a
 //     QuantAct input is copied), so no operand pass runs before it.
 //   * A wave takes its K range a unit (128 or 256 K) at a time, the next unit's weight bytes in flight
@@ -19,7 +20,7 @@
 // afford (ah_gemm.hip's f16 operands fold once a super-block); at one or two token tiles it is a
 // few hundred cycles in all.
 // Measured on MI355X: the FFN of 8 tokens at 1536 / 8960 (Q4_K gate and up, Q6_K down) 53.9 -> 27.7 us
-// in two launches instead of seven; Q5_0 4861 x 901 at 5 tokens 19.3 -> 8.9 us (the host's own rate);
+// in two launches instead of seven; Q5_0 4861 x 901 at 5 tokens 19.4 -> 7.5 us;
 // Q6_K 1536 x 8960 at 16 tokens 33.3 -> 16.6 us from codes.
 #include "ah_internal.h"
 #include "ah_few.h"

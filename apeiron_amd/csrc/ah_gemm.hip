@@ -988,7 +988,8 @@ AH_DEV __attribute__((always_inline)) void gemm_rb_body(GemmArgs a, uint8_t *lds
                              rb::lds_bytes<TYPE, WV, RG>());
 }
 
-// CHUNK false: every part's token tiles are one chunk.  The chunk arithmetic costs a call of one
+// CHUNK false: every part's token tiles are one chunk (a launch with one chunked part runs all its
+// parts chunked; the mixed K-quant and the dequantize-once kernels have the chunked form alone).  The chunk arithmetic costs a call of one
 // chunk 0.1 to 0.3 us, and Q4_K's kernel, with 128 VGPRs and no scalar register to spare, 2 us in
 // spills (8960x1536, 24 tokens: 18.5 us without, 20.0 with).
 template <int TYPE, int WV, int RG, bool CHUNK>
@@ -1936,8 +1937,8 @@ uint32_t per_split(const GemmGeom &g, uint32_t splits) {
 }  // namespace
 
 // Split-K count for an n_tok x n_out GEMM on `cus` compute units.  Cost model (microseconds),
-// fitted to a sweep of every valid split count over the configs[3] and configs[4] prefill shapes
-// at N = 512 on MI355X (it picks the measured best for all 13):
+// fitted to a sweep of every valid split count over the prefill shapes of the models of hidden 896
+// and 1536 at N = 512 on MI355X (it picks the measured best for all 13):
 //   the busiest CU runs ceil(workgroups / cus) workgroups of `per` stages, c_type us a stage
 //   (a second resident Q4_K workgroup shares the CU's throughput rather than adding to it);
 //   a split GEMM adds the reduction: 4.8 us fixed plus the partials' write and read-back,

@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(kThreads)
 // (token, block) advances by a fixed pair with one carry, so no block pays a division.  Against
 // loads and stores of single elements off the 16-byte grid and 64-bit divisions, us for 2048 rows
 // of f32: 8960 columns 17.8 -> 15.6 (6.2 TB/s, part of it from the Infinity Cache), 8957 columns
-// 35.1 -> 15.8, 901 columns 6.2 -> 3.5 (the host's call).
+// 35.1 -> 15.8, 901 columns 6.2 -> 3.5 (calls back to back, nothing else between them on the host).
 template <uint32_t SRC>
 __global__ void __launch_bounds__(kThreads) quant_kernel(QuantArgs q) {
     const uint32_t i0 = blockIdx.x * (kThreads / 4) + threadIdx.x / 4, step = gridDim.x * (kThreads / 4);
@@ -226,7 +226,7 @@ AH_DEV QuadIn operand_load(const ActRsrc &r, uint32_t n_in, uint32_t b) {
 
 // The same for code rows that start at any byte (n_in % 4 != 0): one 8-byte load at the lane's
 // own address where it has 8 codes, single bytes at the row's end.  A load a byte made the whole
-// GEMM of 512 rows x 8957 columns 38.9 us at 512 tokens (now 36.7, as 8960 columns take) and, at
+// Q8_0 GEMM of 512 rows x 8957 columns 38.9 us at 512 tokens (now 36.7, as 8960 columns take) and, at
 // 2048 tokens, 9.7 us slower than 8960 columns (now 1.9).
 AH_DEV QuadIn operand_load_bytes(const int8_t *x, const int64_t *scales, uint32_t n_in, uint32_t b, uint32_t nb32) {
     const uint32_t k0 = b * 32 + 8 * (threadIdx.x & 3);
@@ -474,7 +474,7 @@ AH_DEV GemvPart part_at(const GemvPart *__restrict__ parts, uint32_t i) {
 // LDS: [activation region: act_bytes][one tile slot per wave].
 // Single-type kernels run 4 waves per SIMD (two workgroups per CU, <= 128 VGPRs).  The mixed-type
 // kernel holds every type's unit loop and spilled at that budget (1.1 MB of scratch writes per
-// configs[4] q/k/v launch); its plans are small (36 workgroups for q/k/v), so it is built for 2
+// q/k/v launch at hidden 1536); its plans are small (36 workgroups for q/k/v), so it is built for 2
 // waves per SIMD (one workgroup per CU, <= 256 VGPRs), which costs those plans nothing.
 template <int TYPE>
 constexpr int stream_waves_per_simd() { return TYPE == kMixedType ? 2 : 4; }
@@ -522,8 +522,8 @@ AH_DEV void ffn_epilogue(const FfnArgs &fa, uint32_t b0, uint32_t b1, const floa
 // 32-lane half-wave per (token, hidden block), the wave's two blocks consecutive; refusals keyed
 // past the projections': an element's conversion or SwiGLU at key_sw + t * n_ff + k, a block's
 // quantizer at key_q + t * ceil(n_ff / 32) + b.
-// Bound by its f64 arithmetic (about 130 VALU instructions an element; the 9 bytes an element
-// move faster).  A wave steps by the whole grid, so its (token, block) advances by a fixed pair
+// About 130 VALU instructions an element, most of them f64, issue in some 60 of the 92 us of 2048 x
+// 8960; its 9 bytes an element are 32 us of a copy.  A wave steps by the whole grid, so its (token, block) advances by a fixed pair
 // with one carry instead of a division, and its next two blocks are requested before it computes.
 __global__ void __launch_bounds__(kThreads) swiglu_quant_kernel(SwigluArgs a) {
     const uint32_t nbh = (a.n_ff + 31) / 32;
@@ -1076,7 +1076,7 @@ AH_DEV void seq_swiglu_stage(const SeqArgs &a, uint32_t s, uint32_t r, bool &bro
 }
 
 // Built for 2 waves per SIMD (one resident workgroup per CU, <= 256 VGPRs): at 4 the Q4_K and
-// Q6_K forms spilled ~100 bytes a lane, and the configs[4] token measured the same either way
+// Q6_K forms spilled ~100 bytes a lane, and the token of hidden 1536 measured the same either way
 // (827-829 us).
 template <int TYPE>
 __global__ void __launch_bounds__(kSThreads, 2) gemv_seq_kernel(SeqArgs a) {
@@ -1195,7 +1195,7 @@ int ah_gemv_seq_occupancy(uint32_t type, size_t act_bytes) {
 // One launch runs the whole sequence, its grid at most the workgroups the device holds at once
 // (ah_gemv_seq_occupancy per CU), so on a device the launch has to itself every workgroup is
 // resident, as the grid barriers between stages need.  An ordinary launch, not a cooperative one:
-// it measured 2% faster on the configs[4] token (817 against 835 us), and rocprofv3's kernel trace
+// it measured 2% faster on the token of hidden 1536 (817 against 835 us), and rocprofv3's kernel trace
 // of a process that made cooperative launches ended in a segmentation fault at exit, before it
 // wrote its results, while the same trace with ordinary launches completes.  Should other work
 // hold CUs so that some workgroups start late, the waits are bounded: the run then reports

@@ -186,7 +186,9 @@ int32_t ah_ffn_q8_dev(ah_ctx *ctx, const ah_tensor *gate, const ah_tensor *up, c
  * hold gate and up rows of the same 64 hidden indices, and the epilogue writes the hidden
  * QuantAct (no gate / up matrix in memory) -- the form ah_set_ffn_prefill_form selects with
  * AH_FFN_PREFILL_FUSED; the default (AUTO, and every other type) runs the grouped gate/up GEMM,
- * then a SwiGLU pass (ah_swiglu_quant_dev's kernel), which measured faster on MI355X.
+ * then a SwiGLU pass (ah_swiglu_quant_dev's kernel), which measured faster on MI355X.  Where gate
+ * and up take the few-token kernel (AH_GEMM_DESIGN_AUTO below; rows of up to 3072 columns, 1536 for
+ * Q8_0 and Q5_0), AUTO is one launch of it with the SwiGLU in its epilogue: the same bits.
  * ah_ffn_prefill_dev adds the down projection (n_embd x n_ff, any type) from the hidden QuantAct
  * (d_h_codes 4-byte aligned) into d_y[n_tok][n_embd].  Refusals (ah_sync_status) in the
  * reference FFN's order: the input's quantization, the gate projection's outputs (token-major),
@@ -206,7 +208,7 @@ int32_t ah_ffn_prefill_dev(ah_ctx *ctx, const ah_tensor *gate, const ah_tensor *
 int32_t ah_ffn_prefill_q8_dev(ah_ctx *ctx, const ah_tensor *gate, const ah_tensor *up, const ah_tensor *down,
                               const int8_t *d_codes, const int64_t *d_scales, size_t n_tok, float *d_y,
                               int8_t *d_h_codes, int64_t *d_h_scales, void *stream);
-/* The prefill FFN's form per context: AUTO (the default: two passes), FUSED (one launch for
+/* The prefill FFN's form per context: AUTO (the default: two passes, or a few-token launch), FUSED (one launch for
  * Q4_K / Q2_K / Q3_K gate/up; other types keep two passes) or TWO_PASS.  The hidden QuantAct is
  * bit-identical given the same gate / up values; those agree within the GEMM tolerance. */
 #define AH_FFN_PREFILL_AUTO 0u
@@ -289,8 +291,9 @@ int32_t ah_seq_info(const ah_seq *seq, uint32_t *grid, uint32_t *act_bytes);
 
 /* y[n_tok][n_out] (token-major) = X W^T for X[n_tok][n_in] f32; quantization is a separate
  * in-stream pass into context scratch (grown on demand, never shrunk), which also holds split-K
- * partials.  (Calls of a few tokens quantize inside the kernel where that is cheaper.)  GEMM calls on one context share that scratch: calls on different streams of the same
- * context must not overlap (use one context per stream for concurrent prefills). */
+ * partials.  (Calls of a few tokens quantize inside the kernel where that is cheaper.)  GEMM calls
+ * on one context share that scratch: calls on different streams of the same context must not
+ * overlap (use one context per stream for concurrent prefills). */
 int32_t ah_gemm_f32_dev(ah_ctx *ctx, const ah_tensor *w, const float *d_x, size_t n_tok,
                         float *d_y, void *stream);
 /* ah_gemm_f32_dev that allocates nothing.  No counterpart in the reference: it is for callers
@@ -321,16 +324,20 @@ int32_t ah_gemm_q8_dev(ah_ctx *ctx, const ah_tensor *w, const int8_t *d_codes,
  *     the dots are per 32-element sub-block on the raw nibbles, folded with d sc_j and, for the
  *     min term, dmin m_j times the token's scaled code sum (two more bf16 outer products);
  *   AH_GEMM_DESIGN_F16: v_mfma_f32_32x32x16_f16 on exact f16 operands (the K-quants' design);
- *   AH_GEMM_DESIGN_AUTO (the default): the F16 design, measured 17-25% faster on MI355X at the
- *     configs[3] shapes (N = 512); up to 32 tokens, where the activations fit a CU's LDS, a
- *     one-launch kernel of its own (int8 block dots folded per block as the GEMV folds them).
+ *   AH_GEMM_DESIGN_AUTO (the default): the F16 design, measured 17-25% faster than INT8 on MI355X at
+ *     512 tokens of 4864x896, 896x4864, 8960x1536 and 1536x8960.  Up to 32 tokens a one-launch
+ *     kernel of its own (int8 block dots folded per block as the GEMV folds them), where the
+ *     activations fit a CU's LDS and that kernel is the faster one: not for wide projections of
+ *     long rows, and past 16 tokens for Q4_K and Q2_K only where two workgroups of 16 tokens for
+ *     each group of rows fit the CUs.  A call's route depends on its projection and token count
+ *     alone (a call whose outputs lie over its input keeps the F16 design).
  *   AH_GEMM_DESIGN_F16_TILE: the dequantize-once design for Q4_K, Q2_K and Q3_K: each 256-thread
  *     workgroup owns a 128-row x 128-token tile, converts each weight super-block to exact f16
  *     (sc * q, folded with d and the min term per super-block) once into LDS, and every wave
  *     feeds v_mfma_f32_32x32x16_f16 from that LDS copy and from activation fragments in
  *     registers.
- * Per type: Q8_0 takes AUTO, F16 or INT8; Q4_K takes AUTO (= F16), F16, INT8 or F16_TILE; Q2_K and
- * Q3_K take AUTO (= F16_TILE) or F16, which for these two types serves the prefill as one
+ * Per type: Q8_0 takes AUTO, F16 or INT8; Q4_K takes AUTO, F16, INT8 or F16_TILE; Q2_K and Q3_K
+ * take AUTO (past a few tokens F16_TILE), F16_TILE or F16, which for these two types serves the prefill as one
  * streaming GEMV per token (the reference's matmat_q8act loop, chart/mod.rs:1955-1975); Q5_0,
  * Q6_K and Q8_K take AUTO or F16.  Any other pairing returns AH_ERR_UNSUPPORTED_QUANT. */
 #define AH_GEMM_DESIGN_AUTO 0u

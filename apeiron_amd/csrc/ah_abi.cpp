@@ -534,8 +534,11 @@ uint32_t few_tok_tile(const ah_ctx *ctx, const ah_tensor *t, size_t n_tok) {
     const double cost = ah_few_cost(t->type, n_in, kpad, n < run ? n : run, splits, few_waves(splits), wgs * ((n + run - 1) / run), cus);
     if (cost > 0.0) {
         double tile = 0.0;
-        ah_gemm_pick_splits(t->type, (uint32_t)t->n_out, n_in, n, cus, ah_k23((int)t->type) ? kGemmKindTile : kGemmKindRb, &tile);
-        if (cost > 8.6 + 0.78 * tile) return 0;
+        const uint32_t s = ah_gemm_pick_splits(t->type, (uint32_t)t->n_out, n_in, n, cus,
+                                               ah_k23((int)t->type) ? kGemmKindTile : kGemmKindRb, &tile);
+        // (a plan whose partials would fill the no-alloc form's scratch stays here, where it needs none)
+        const bool fits = s == 1 || (size_t)s * n * t->n_out * 4 <= kNoAllocScratchBytes / 2;
+        if (fits && cost > 8.6 + 0.78 * tile) return 0;
     }
     return tok;
 }
